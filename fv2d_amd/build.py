@@ -4,7 +4,9 @@
 
 The FP64 stage and the C-ABI layer are compiled with -ffp-contract=off (no a*b+c
 contraction into FMA), which keeps the FP64 path bit-identical to the reference's
-arithmetic. The FP32-form stage may contract. All HIP code is built with the packed-FP32
+arithmetic. The FP32-form stage may contract
+within an expression (-ffp-contract=on), so that every kernel of a class (march and strip, single
+and batched) fuses the same operations and gives the same bits. All HIP code is built with the packed-FP32
 target feature disabled.
 """
 from __future__ import annotations
@@ -35,7 +37,12 @@ COMMON = [
 UNITS = [
     ("stage_fp64.hip", ["-ffp-contract=off"]),
     ("stage_fp64_exact.hip", ["-ffp-contract=off"]),
-    ("stage_fp32.hip", ["-ffp-contract=fast"]),
+    ("stage_fp32.hip", ["-ffp-contract=on"]),
+    ("march_fp64.hip", ["-ffp-contract=off"]),
+    ("march_fp64_exact.hip", ["-ffp-contract=off"]),
+    ("march_fp32.hip", ["-ffp-contract=on"]),
+    ("march_batch_fp64.hip", ["-ffp-contract=off"]),
+    ("march_batch_fp32.hip", ["-ffp-contract=on"]),
     ("fv2d_capi.hip", ["-ffp-contract=off"]),
     ("fv2d_batch.hip", ["-ffp-contract=off"]),
     ("fv2d_noalloc.hip", ["-ffp-contract=off"]),

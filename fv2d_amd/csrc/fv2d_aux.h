@@ -33,10 +33,11 @@ __global__ void init_state_kernel(KParams kp, const double *q, S *U, S *Q0) {
 }
 
 // Max hyperbolic inverse dt over Q0 or over reset(consToPrim(U)): workgroup b covers a
-// contiguous run of cells and writes partials[b] (the stage epilogue's partial layout).
+// contiguous run of cells and writes partials[b] (the strip kernel's partial layout), or joins
+// the march kernel's slots when acc is given.
 template <typename R, typename S>
 __global__ void __launch_bounds__(256) dt_cells_kernel(KParams kp, const S *src, int from_q0, double *partials,
-                                                       int nparts) {
+                                                       int nparts, unsigned long long *acc) {
   const long long n = (long long)kp.Nx * kp.Ny;
   const long long per = (n + nparts - 1) / nparts;
   const long long c0 = blockIdx.x * per;
@@ -59,7 +60,12 @@ __global__ void __launch_bounds__(256) dt_cells_kernel(KParams kp, const S *src,
   m = wave_max(m);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
-  if (threadIdx.x == 0) partials[blockIdx.x] = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+  if (threadIdx.x != 0) return;
+  const double b = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+  if (acc)
+    acc_max(acc, blockIdx.x, b);
+  else
+    partials[blockIdx.x] = b;
 }
 
 // Loop control of main.cpp:62-83 for one step, given the reduced hyperbolic inverse dt:
@@ -100,7 +106,23 @@ static __global__ __attribute__((unused)) void __launch_bounds__(1024) reduce_ke
   if (advance) advance_control(ctl, b, kp, dts_log);
 }
 
-static __global__ __attribute__((unused)) void set_dt_kernel(StepCtl *ctl, double dt, double dx, double dy) {
+// The same for the march kernel (one wave): its slots keep the maximum of the current state
+// until a step that replaces the state begins.
+static __global__ __attribute__((unused)) void __launch_bounds__(64) reduce_acc_kernel(StepCtl *ctl, unsigned long long *acc, KParams kp,
+                                                              int advance, double *dts_log) {
+  const double b = acc_read(acc);
+  const bool was = ctl->active != 0;
+  if (threadIdx.x == 0) {
+    ctl->inv_hyp = b;
+    if (advance && was) advance_control(ctl, b, kp, dts_log);
+  }
+  __syncthreads();
+  if (advance && was && ctl->active) acc_clear(acc);
+}
+
+static __global__ __attribute__((unused)) void __launch_bounds__(64) set_dt_kernel(StepCtl *ctl, unsigned long long *acc, double dt, double dx, double dy) {
+  if (acc) acc_clear(acc);
+  if (threadIdx.x != 0) return;
   ctl->dt = dt;
   ctl->dt_dx = dt / dx;
   ctl->dt_dy = dt / dy;
@@ -115,7 +137,9 @@ static __global__ __attribute__((unused)) void set_loop_kernel(StepCtl *ctl, dou
   ctl->active = 1;
 }
 
-static __global__ __attribute__((unused)) void clear_ctl_kernel(StepCtl *ctl) {
+static __global__ __attribute__((unused)) void __launch_bounds__(64) clear_ctl_kernel(StepCtl *ctl, unsigned long long *acc) {
+  if (acc) acc_clear(acc);
+  if (threadIdx.x != 0) return;
   ctl->dt = ctl->dt_dx = ctl->dt_dy = 0.0;
   ctl->t = ctl->tend = 0.0;
   ctl->inv_hyp = 0.0;

@@ -32,6 +32,7 @@
 #include "../../include/fv2d_amd.h"
 #include "fv2d_aux.h"
 #include "fv2d_device.h"
+#include "fv2d_march_device.h"
 #include "fv2d_params.h"
 
 using namespace fv2d;
@@ -44,11 +45,28 @@ constexpr size_t ARENA_ALIGN = 256;
 
 // ------------------------------------------------------------------ device kernels
 
+// Loop control of each running job of march class `cls` for its next step, one wave per slot.
+// Workgroup 0 also clears the class's work-list counters that this step's stage kernels start from.
+__global__ void __launch_bounds__(64) batch_control_kernel(const BatchJob *jobs, int *counters, int cls) {
+  if (blockIdx.x == 0 && threadIdx.x < 16)
+    counters[2 * cls * COUNTER_WORDS + (int)threadIdx.x * COUNTER_STRIDE] = 0;
+  const BatchJob &J = jobs[blockIdx.x];
+  if (!J.used || J.cls != cls) return;
+  StepCtl *ctl = J.ctl;
+  if (!ctl->active) return;
+  const double b = acc_read(J.acc);
+  acc_clear(J.acc);
+  if (threadIdx.x != 0) return;
+  ctl->inv_hyp = b;
+  if (ctl->nsteps > 0) ctl->fresh = 0;  // the first step reads Q0, later ones reset(c2p(U))
+  advance_control(ctl, b, J.kp, nullptr);
+}
+
 // One workgroup per slot: reduce the dt partials of each running job of class `cls` and run
 // its loop control (the single-simulation reduce_kernel in advance mode). Workgroup 0 also
 // clears the class's work-list counters that this step's stage kernels start from.
 __global__ void __launch_bounds__(256) batch_reduce_kernel(const BatchJob *jobs, int *counters, int cls) {
-  if (blockIdx.x == 0 && threadIdx.x < 2) counters[2 * cls + threadIdx.x] = 0;
+  if (blockIdx.x == 0 && threadIdx.x < 2) counters[(2 * cls + threadIdx.x) * COUNTER_WORDS] = 0;
   const BatchJob &J = jobs[blockIdx.x];
   if (!J.used || J.cls != cls) return;
   StepCtl *ctl = J.ctl;
@@ -66,8 +84,8 @@ __global__ void __launch_bounds__(256) batch_reduce_kernel(const BatchJob *jobs,
   advance_control(ctl, b, J.kp, nullptr);
 }
 
-// Work list: for each class c, the items (slot, segment) of every used, running job of
-// class c, in slot order, at items[ranges[2c] .. ranges[2c] + ranges[2c+1]).
+// Work list: for each class c, the items (slot, segment; march classes: slot, group of tasks) of
+// every used, running job of class c, in slot order, at items[ranges[2c] .. ranges[2c] + ranges[2c+1]).
 __global__ void __launch_bounds__(1024) pack_items_kernel(const BatchJob *jobs, int nslots, int nclasses,
                                                           BatchItem *items, int *ranges) {
   __shared__ int cnt[MAX_SLOTS];
@@ -77,7 +95,8 @@ __global__ void __launch_bounds__(1024) pack_items_kernel(const BatchJob *jobs, 
     int n = 0;
     if (c < nclasses && s < nslots) {
       const BatchJob &J = jobs[s];
-      if (J.used && J.cls == c && J.ctl->active) n = J.nblocks;
+      if (J.used && J.cls == c && J.ctl->active)
+        n = J.march ? (J.nblocks + MARCH_GROUP - 1) / MARCH_GROUP : J.nblocks;
     }
     cnt[s] = n;
     __syncthreads();
@@ -112,7 +131,9 @@ __global__ void drop_job_kernel(BatchJob *jobs, int slot) {
 }
 
 // A new job's control block: t = 0, loop to (tend, max_steps), first step from Q0.
-__global__ void init_job_ctl_kernel(StepCtl *ctl, double tend, int max_steps) {
+__global__ void init_job_ctl_kernel(StepCtl *ctl, unsigned long long *acc, double tend, int max_steps) {
+  acc_clear(acc);
+  if (threadIdx.x != 0) return;
   ctl->dt = ctl->dt_dx = ctl->dt_dy = 0.0;
   ctl->t = 0.0;
   ctl->tend = tend;
@@ -147,7 +168,8 @@ struct JobLayout {
 
 size_t align_up(size_t x) { return (x + ARENA_ALIGN - 1) / ARENA_ALIGN * ARENA_ALIGN; }
 
-// Rows per chunk of a batched job: its own chunk_rows, else 4.
+// Rows per chunk of a batched job on the strip kernel: its own chunk_rows, else 4. The job's arena
+// layout and its share of max_items follow the strip kernel's split for both kernels.
 int batch_chunk_rows(const fv2d_params *p) { return p->chunk_rows > 0 ? p->chunk_rows : CHUNK_ROWS_DEFAULT; }
 
 int batch_seg_rows(const fv2d_params *p) {
@@ -161,6 +183,14 @@ int batch_seg_rows(const fv2d_params *p) {
 
 StripGeom batch_geom(const fv2d_params *p) {
   return strip_geom(p->Nx, p->Ny, batch_seg_rows(p), batch_chunk_rows(p));
+}
+
+// The march kernel's split (jobs without chunk_rows): tasks of 16 rows by default. Its items of
+// MARCH_GROUP tasks are then never more than the strip split's (at most twice the strips, four
+// times the segments).
+bool batch_march(const fv2d_params *p) { return p->chunk_rows <= 0; }
+MarchGeom batch_march_geom(const fv2d_params *p) {
+  return march_geom(p->Nx, p->Ny, p->seg_rows > 0 ? p->seg_rows : 16);
 }
 
 JobLayout job_layout(const fv2d_params *p) {
@@ -182,7 +212,7 @@ StageClass class_of(const fv2d_params &p, const KParams &kp) {
   c.tc = p.tc_active ? 1 : 0;
   c.visc = p.visc_active ? 1 : 0;
   c.xg = needs_xg(kp) ? 1 : 0;
-  c.nw = batch_chunk_rows(&p);
+  c.nw = batch_march(&p) ? 0 : batch_chunk_rows(&p);
   return c;
 }
 
@@ -198,6 +228,7 @@ struct fv2d_batch {
   std::map<size_t, size_t> free_ranges;  // offset -> size, coalesced
   BatchJob *d_jobs = nullptr;
   StepCtl *d_ctl = nullptr;
+  unsigned long long *d_acc = nullptr;  // per slot: the march kernel's dt slots (ACC_WORDS)
   BatchItem *d_items = nullptr;
   int *d_ranges = nullptr;
   int *d_counters = nullptr;
@@ -299,12 +330,15 @@ static int class_index(fv2d_batch *b, const StageClass &c) {
 
 // One step of the jobs of class c on stream st: reduce + loop control, stage 1, stage 2.
 static hipError_t enqueue_class_step(fv2d_batch *b, int c, hipStream_t st) {
-  hipLaunchKernelGGL(batch_reduce_kernel, dim3(b->cfg.max_jobs), dim3(256), 0, st, b->d_jobs, b->d_counters, c);
+  if (b->classes[c].nw == 0)
+    hipLaunchKernelGGL(batch_control_kernel, dim3(b->cfg.max_jobs), dim3(64), 0, st, b->d_jobs, b->d_counters, c);
+  else
+    hipLaunchKernelGGL(batch_reduce_kernel, dim3(b->cfg.max_jobs), dim3(256), 0, st, b->d_jobs, b->d_counters, c);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const bool f32 = b->cfg.precision == FV2D_FP32;
   for (int stage = 1; stage <= 2; ++stage) {
-    int *counter = b->d_counters + 2 * c + (stage - 1);
+    int *counter = b->d_counters + (2 * c + (stage - 1)) * COUNTER_WORDS;
     const int *range = b->d_ranges + 2 * c;
     e = f32 ? launch_batch_fp32(b->classes[c], b->d_jobs, b->d_items, range, counter, stage, b->grid[c], st)
             : launch_batch_fp64(b->classes[c], b->d_jobs, b->d_items, range, counter, stage, b->grid[c], st);
@@ -399,7 +433,7 @@ void fv2d_batch_destroy(fv2d_batch *b) {
     if (e) (void)hipEventDestroy(e);
   for (hipEvent_t e : b->cls_join) (void)hipEventDestroy(e);
   for (hipStream_t st : b->cls_stream) (void)hipStreamDestroy(st);
-  void *bufs[] = {b->arena, b->d_jobs, b->d_ctl, b->d_items, b->d_ranges, b->d_counters,
+  void *bufs[] = {b->arena, b->d_jobs, b->d_ctl, b->d_acc, b->d_items, b->d_ranges, b->d_counters,
                   b->d_upload, b->d_out, b->d_rowsum, b->d_sums};
   for (void *x : bufs)
     if (x) (void)hipFree(x);
@@ -456,10 +490,12 @@ int fv2d_batch_create(const fv2d_batch_config *c, fv2d_batch **out) {
   b->free_ranges[0] = (size_t)b->cfg.arena_bytes;
   if ((e = hipMalloc((void **)&b->d_jobs, sizeof(BatchJob) * c->max_jobs)) != hipSuccess) return fail("jobs", e);
   if ((e = hipMalloc((void **)&b->d_ctl, sizeof(StepCtl) * c->max_jobs)) != hipSuccess) return fail("ctl", e);
+  if ((e = hipMalloc((void **)&b->d_acc, sizeof(unsigned long long) * ACC_WORDS * c->max_jobs)) != hipSuccess)
+    return fail("dt slots", e);
   if ((e = hipMalloc((void **)&b->d_items, sizeof(BatchItem) * (size_t)c->max_items)) != hipSuccess)
     return fail("work list", e);
   if ((e = hipMalloc((void **)&b->d_ranges, sizeof(int) * 2 * MAX_CLASSES)) != hipSuccess) return fail("ranges", e);
-  if ((e = hipMalloc((void **)&b->d_counters, sizeof(int) * 2 * MAX_CLASSES)) != hipSuccess)
+  if ((e = hipMalloc((void **)&b->d_counters, sizeof(int) * 2 * MAX_CLASSES * COUNTER_WORDS)) != hipSuccess)
     return fail("counters", e);
   if ((e = hipMalloc((void **)&b->d_sums, sizeof(double) * 4)) != hipSuccess) return fail("sums", e);
   if ((e = hipHostMalloc((void **)&b->h_ctl, sizeof(StepCtl) * c->max_jobs, hipHostMallocDefault)) != hipSuccess)
@@ -472,7 +508,7 @@ int fv2d_batch_create(const fv2d_batch_config *c, fv2d_batch **out) {
     return fail("clear ctl", e);
   if ((e = hipMemsetAsync(b->d_ranges, 0, sizeof(int) * 2 * MAX_CLASSES, b->stream)) != hipSuccess)
     return fail("clear ranges", e);
-  if ((e = hipMemsetAsync(b->d_counters, 0, sizeof(int) * 2 * MAX_CLASSES, b->stream)) != hipSuccess)
+  if ((e = hipMemsetAsync(b->d_counters, 0, sizeof(int) * 2 * MAX_CLASSES * COUNTER_WORDS, b->stream)) != hipSuccess)
     return fail("clear counters", e);
   hipEvent_t *evs[] = {&b->ev_start, &b->ev_end, &b->ev_ctl, &b->ev_upload};
   for (hipEvent_t *ev : evs)
@@ -533,6 +569,7 @@ int fv2d_batch_submit(fv2d_batch *b, const fv2d_params *p, const fv2d_problem *p
   J.partials = (double *)(base + 3 * L.state);
   J.grav_row = L.grav ? (float *)(base + 3 * L.state + L.partials) : nullptr;
   StepCtl *ctl = b->d_ctl + slot;
+  unsigned long long *slot_acc = b->d_acc + (size_t)slot * ACC_WORDS;
   const long long n = (long long)p->Nx * p->Ny;
   const bool f32 = b->cfg.precision == FV2D_FP32;
 
@@ -579,13 +616,14 @@ int fv2d_batch_submit(fv2d_batch *b, const fv2d_params *p, const fv2d_problem *p
                          (double *)J.U, (double *)J.Q0);
   }
   BHIP(b, hipGetLastError());
-  hipLaunchKernelGGL(init_job_ctl_kernel, dim3(1), dim3(1), 0, b->stream, ctl, tend, max_steps);
+  hipLaunchKernelGGL(init_job_ctl_kernel, dim3(1), dim3(64), 0, b->stream, ctl, slot_acc, tend, max_steps);
+  unsigned long long *acc = batch_march(p) ? slot_acc : nullptr;
   if (f32)
     hipLaunchKernelGGL((dt_cells_kernel<float, float>), dim3(J.g.nblocks), dim3(256), 0, b->stream, J.kp,
-                       (const float *)J.Q0, 1, J.partials, J.g.nblocks);
+                       (const float *)J.Q0, 1, J.partials, J.g.nblocks, acc);
   else
     hipLaunchKernelGGL((dt_cells_kernel<double, double>), dim3(J.g.nblocks), dim3(256), 0, b->stream, J.kp,
-                       (const double *)J.Q0, 1, J.partials, J.g.nblocks);
+                       (const double *)J.Q0, 1, J.partials, J.g.nblocks, acc);
   BatchJob dj;
   memset(&dj, 0, sizeof dj);
   dj.kp = J.kp;
@@ -593,12 +631,21 @@ int fv2d_batch_submit(fv2d_batch *b, const fv2d_params *p, const fv2d_problem *p
   dj.seg = J.g.seg;
   dj.nsx = J.g.nsx;
   dj.nsy = J.g.nsy;
+  if (batch_march(p)) {
+    const MarchGeom mg = batch_march_geom(p);
+    dj.nblocks = mg.ntasks;
+    dj.seg = mg.seg;
+    dj.nsx = mg.nsx;
+    dj.nsy = mg.nsy;
+    dj.march = 1;
+  }
   dj.U = J.U;
   dj.Us = J.Us;
   dj.Q0 = J.Q0;
   dj.grav_row = J.grav_row;
   dj.ctl = ctl;
   dj.partials = J.partials;
+  dj.acc = slot_acc;
   dj.rk2 = (p->time_stepping == FV2D_TS_RK2) ? 1 : 0;
   dj.used = 1;
   dj.cls = cls;

@@ -176,8 +176,7 @@ int fv2d_create(const fv2d_params *p, fv2d_handle **out) {
   h->esize = (p->precision == FV2D_FP32) ? 4 : 8;
   const int pitch = (p->Nx + 63) / 64 * 64;
   build_kparams(p, pitch, h->d.kp);
-  h->d.geom = sim_geom(p);
-  h->d.nparts = h->d.geom.nblocks;
+  sim_set_geom(h->d);
 
   auto fail = [&](const char *what, hipError_t e) {
     char b[512];
@@ -194,7 +193,7 @@ int fv2d_create(const fv2d_params *p, fv2d_handle **out) {
   if ((e = hipMalloc(&h->d.Us, state_bytes)) != hipSuccess) return fail("hipMalloc Us", e);
   if ((e = hipMalloc(&h->d.Q0, state_bytes)) != hipSuccess) return fail("hipMalloc Q0", e);
   if ((e = hipMalloc((void **)&h->d.ctl, sizeof(StepCtl))) != hipSuccess) return fail("hipMalloc ctl", e);
-  if ((e = hipMalloc((void **)&h->d.partials, sizeof(double) * h->d.nparts)) != hipSuccess)
+  if ((e = hipMalloc((void **)&h->d.partials, sim_partials_bytes(h->d))) != hipSuccess)
     return fail("hipMalloc partials", e);
   if ((e = hipMalloc((void **)&h->rowsum, sizeof(double) * 4 * (size_t)p->Ny)) != hipSuccess)
     return fail("hipMalloc rowsum", e);
@@ -210,7 +209,7 @@ int fv2d_create(const fv2d_params *p, fv2d_handle **out) {
     if (e != hipSuccess) return fail("gravity table", e);
     h->d.grav_row = h->grav_tab;
   }
-  hipLaunchKernelGGL(clear_ctl_kernel, dim3(1), dim3(1), 0, h->d.stream, h->d.ctl);
+  hipLaunchKernelGGL(clear_ctl_kernel, dim3(1), dim3(64), 0, h->d.stream, h->d.ctl, sim_acc(h->d));
   if ((e = hipStreamSynchronize(h->d.stream)) != hipSuccess) return fail("init", e);
   *out = h;
   return FV2D_OK;
@@ -237,7 +236,7 @@ int fv2d_set_prim(fv2d_handle *h, const double *q) {
     hipLaunchKernelGGL(init_state_kernel<double>, dim3(grid_1d(n)), dim3(AUX_THREADS), 0, h->d.stream, h->d.kp,
                        h->staging, (double *)h->d.U, (double *)h->d.Q0);
   HIPH(h, hipGetLastError());
-  hipLaunchKernelGGL(clear_ctl_kernel, dim3(1), dim3(1), 0, h->d.stream, h->d.ctl);
+  hipLaunchKernelGGL(clear_ctl_kernel, dim3(1), dim3(64), 0, h->d.stream, h->d.ctl, sim_acc(h->d));
   SIMH(h, sim_launch_dt_tiles(h->d, h->d.Q0, 1));
   SIMH(h, sim_launch_reduce(h->d, 0, nullptr));
   HIPH(h, hipStreamSynchronize(h->d.stream));
@@ -261,7 +260,7 @@ int fv2d_set_problem(fv2d_handle *h, const fv2d_problem *prob) {
     hipLaunchKernelGGL(problem_ic_kernel<double>, dim3(grid_1d(n)), dim3(AUX_THREADS), 0, h->d.stream, h->d.kp, a,
                        (double *)h->d.U, (double *)h->d.Q0);
   HIPH(h, hipGetLastError());
-  hipLaunchKernelGGL(clear_ctl_kernel, dim3(1), dim3(1), 0, h->d.stream, h->d.ctl);
+  hipLaunchKernelGGL(clear_ctl_kernel, dim3(1), dim3(64), 0, h->d.stream, h->d.ctl, sim_acc(h->d));
   SIMH(h, sim_launch_dt_tiles(h->d, h->d.Q0, 1));
   SIMH(h, sim_launch_reduce(h->d, 0, nullptr));
   HIPH(h, hipStreamSynchronize(h->d.stream));
@@ -305,7 +304,7 @@ int fv2d_step(fv2d_handle *h, double dt, fv2d_step_stats *stats) {
   if (!h) return FV2D_E_INVALID;
   if (!h->have_state) FAILH(h, FV2D_E_STATE, "fv2d_step: no state (call fv2d_set_prim first)");
   HIPH(h, hipSetDevice(h->device));
-  hipLaunchKernelGGL(set_dt_kernel, dim3(1), dim3(1), 0, h->d.stream, h->d.ctl, dt, h->d.kp.dx, h->d.kp.dy);
+  hipLaunchKernelGGL(set_dt_kernel, dim3(1), dim3(64), 0, h->d.stream, h->d.ctl, sim_acc(h->d), dt, h->d.kp.dx, h->d.kp.dy);
   HIPH(h, hipGetLastError());
   bool swapped;
   int rc;

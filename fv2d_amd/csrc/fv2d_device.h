@@ -29,6 +29,16 @@ __device__ inline double wave_max(double m) {
   return m;
 }
 
+// The march kernel's dt reduction (ACC_SLOTS): m of task t joins in; the maximum over the slots,
+// by one wave (lane l reads slot l).
+__device__ inline void acc_max(unsigned long long *acc, int t, double m) {
+  atomicMax(acc + (t % ACC_SLOTS) * ACC_STRIDE, (unsigned long long)__double_as_longlong(m));
+}
+__device__ inline double acc_read(const unsigned long long *acc) {
+  return wave_max(__longlong_as_double((long long)acc[(threadIdx.x & 63) * ACC_STRIDE]));
+}
+__device__ inline void acc_clear(unsigned long long *acc) { acc[(threadIdx.x & 63) * ACC_STRIDE] = 0ull; }
+
 // Epilogue commit: reset counters (rare, atomics) and the workgroup's max inverse dt into
 // partials[blk] (no atomics on the hot value: the reduction kernel reads all partials).
 template <int NT>
@@ -138,10 +148,31 @@ strip_kernel(const KParams kp, const StageIO<S> io, const StripGeom g) {
   strip_block<K, R, S>(kp, io, g, blockIdx.x, uni(ctl->dt), uni(ctl->dt_dx), uni(ctl->dt_dy), sm);
 }
 
+// Buffers of a batched job's stage (1 or 2; an Euler job does its whole step in stage 1, with
+// U / Us alternating by step parity; nsteps counts the step being taken).
+template <typename S>
+__device__ inline StageIO<S> batch_stage_io(const BatchJob &J, int stage, int fresh, int nsteps) {
+  // one assignment per field: branches that fill the struct leave it in scratch memory, its
+  // pointers no longer uniform
+  const bool second = J.rk2 && stage == 2;
+  const bool from_u = J.rk2 ? !second : ((nsteps - 1) & 1) == 0;
+  StageIO<S> io;
+  io.src = (const S *)(from_u ? J.U : J.Us);
+  io.out = (S *)(from_u ? J.Us : J.U);
+  io.avg = second ? (const S *)J.U : nullptr;
+  io.q0 = (const S *)J.Q0;
+  io.grav_row = J.grav_row;
+  io.ctl = J.ctl;
+  io.partials = J.partials;
+  io.acc = J.acc;
+  io.qsrc = second ? QSRC_U : (fresh ? QSRC_Q0 : QSRC_U_RESET);
+  io.epilogue = second || !J.rk2;
+  return io;
+}
+
 // Batched stage: a persistent grid pulls (job, item) pairs of one kernel class from its run
 // [range[0], range[0] + range[1]) of the work list through an atomic counter and runs strip_block on them with each job's own
-// parameters, buffers and dt. stage = 1 or 2 (RK2); an Euler job does its whole step in
-// stage 1, with U / Us alternating by step parity. A job's arithmetic does not depend on
+// parameters, buffers and dt. stage = 1 or 2 (batch_stage_io). A job's arithmetic does not depend on
 // the other jobs, so it is bitwise the same alone or in the mix.
 template <class K, typename R, typename S>
 __global__ void __launch_bounds__(K::NT) __attribute__((amdgpu_waves_per_eu(FV2D_WPE_BATCH(K))))
@@ -162,33 +193,7 @@ batch_stage_kernel(const BatchJob *__restrict__ jobs, const BatchItem *__restric
     if (!uni(ctl->active)) continue;
     const int fresh = uni(ctl->fresh), nsteps = uni(ctl->nsteps);
     if (!J.rk2 && stage == 2) continue;
-    StageIO<S> io;
-    io.q0 = (const S *)J.Q0;
-    io.grav_row = J.grav_row;
-    io.ctl = ctl;
-    io.partials = J.partials;
-    if (J.rk2) {
-      if (stage == 1) {
-        io.src = (const S *)J.U;
-        io.qsrc = fresh ? QSRC_Q0 : QSRC_U_RESET;
-        io.avg = nullptr;
-        io.out = (S *)J.Us;
-        io.epilogue = 0;
-      } else {
-        io.src = (const S *)J.Us;
-        io.qsrc = QSRC_U;
-        io.avg = (const S *)J.U;
-        io.out = (S *)J.U;
-        io.epilogue = 1;
-      }
-    } else {
-      const bool odd = ((nsteps - 1) & 1) != 0;  // nsteps counts the step being taken
-      io.src = (const S *)(odd ? J.Us : J.U);
-      io.out = (S *)(odd ? J.U : J.Us);
-      io.qsrc = fresh ? QSRC_Q0 : QSRC_U_RESET;
-      io.avg = nullptr;
-      io.epilogue = 1;
-    }
+    const StageIO<S> io = batch_stage_io<S>(J, stage, fresh, nsteps);
     StripGeom g;
     g.nsx = J.nsx;
     g.nsy = J.nsy;
@@ -201,7 +206,12 @@ batch_stage_kernel(const BatchJob *__restrict__ jobs, const BatchItem *__restric
   }
 }
 
-// Kernel class of a simulation: the template switches of the stage and the chunk height.
+// Work-list counters of a class: 8 per stage (one per XCD for the march kernel; the strip kernel uses
+// the first), each in a cache line of its own.
+constexpr int COUNTER_STRIDE = 32, COUNTER_WORDS = 8 * COUNTER_STRIDE;
+
+// Kernel class of a simulation: the template switches of the stage and the chunk height (nw = 0:
+// the march kernel).
 struct StageClass {
   int recon, riem, tc, visc, xg, nw;
   bool operator==(const StageClass &o) const {
@@ -329,6 +339,13 @@ hipError_t launch_batch_fp32(const StageClass &c, const BatchJob *jobs, const Ba
                              int *counter, int stage, int grid, hipStream_t st);
 int batch_occupancy_fp64(const StageClass &c);
 int batch_occupancy_fp32(const StageClass &c);
+// Their march classes (nw = 0): march_batch_fp64.hip / march_batch_fp32.hip.
+hipError_t launch_batch_march_fp64(const StageClass &c, const BatchJob *jobs, const BatchItem *items, const int *range,
+                                   int *counter, int stage, int grid, hipStream_t st);
+hipError_t launch_batch_march_fp32(const StageClass &c, const BatchJob *jobs, const BatchItem *items, const int *range,
+                                   int *counter, int stage, int grid, hipStream_t st);
+int batch_occupancy_march_fp64(const StageClass &c);
+int batch_occupancy_march_fp32(const StageClass &c);
 hipError_t launch_stage_fp64(const KParams &kp, const StageIO<double> &io, const StripGeom &g, int recon, int riem,
                              bool tc, bool visc, hipStream_t st);
 hipError_t launch_stage_fp64_exact(const KParams &kp, const StageIO<double> &io, const StripGeom &g, int recon,

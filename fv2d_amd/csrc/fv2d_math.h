@@ -134,17 +134,28 @@ struct Ops<float> {
 // r = v_rcp_f64(ds), two Newton steps on r (4 FMAs), then ns = v_div_scale(a), m = ns * r,
 // one FMA correction, v_div_fmas and v_div_fixup. The first half sees a only through the
 // scaling of b, which is the identity unless a, b or a / b lie near the ends of the exponent
-// range. DivBy runs it once for the first numerator; for each further numerator it
-// recomputes the scaled divisor (one instruction) and reuses the refined reciprocal when the
-// two are bitwise equal, so every quotient has the bits of a / b (and is a / b when they
-// differ). On the host and in the FP32 form (where division is a * rcp(b), the reciprocal
-// shared by the compiler) it is plain division.
+// range. DivBy runs it once, for a base numerator; for each further numerator it recomputes the
+// scaled divisor (one instruction) and reuses the refined reciprocal when the two are bitwise
+// equal, so every quotient has the bits of a / b (and is a / b when they differ).
+// v_div_scale gives NaN for a zero or NaN operand, and v_div_fixup then sets the quotient from a
+// and b alone (signed zeros, infinities, NaNs): such a numerator also takes the short way. That
+// matters wherever a velocity is exactly zero (gas at rest, flow along one axis): sent to a / b
+// there, the quotients made the point blast's FP64 stage 14% slower.
+// On the host and in the FP32 form (where division is a * rcp(b), the reciprocal shared by the
+// compiler) it is plain division.
 template <typename R>
 struct DivBy {
   R b, a0;
   FV2D_HD DivBy(R b_, R a0_) : b(b_), a0(a0_) {}
+  FV2D_HD explicit DivBy(R b_) : b(b_), a0(b_) {}
   FV2D_HD R first() const { return Ops<R>::div(a0, b); }
   FV2D_HD R operator()(R a) const { return Ops<R>::div(a, b); }
+  FV2D_HD R maybe_zero(R a) const { return Ops<R>::div(a, b); }
+  template <int N>
+  FV2D_HD void all(const R a[N], R q[N]) const {
+#pragma unroll
+    for (int k = 0; k < N; ++k) q[k] = Ops<R>::div(a[k], b);
+  }
 };
 
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -158,6 +169,12 @@ struct DivBy<double> {
     const double r1 = fma(r, fma(-ds, r, 1.0), r);
     rf = fma(r1, fma(-ds, r1, 1.0), r1);
   }
+  // no base numerator: the scaling of b / b (ds is NaN only for a zero or NaN divisor)
+  __device__ explicit DivBy(double b_) : DivBy(b_, b_) {}
+  __device__ double scaled(double a) const {
+    bool scale;
+    return __builtin_amdgcn_div_scale(a, b, false, &scale);
+  }
   // the second half of the division, for a numerator whose scaled divisor is ds
   __device__ double quot(double a) const {
     bool scale;
@@ -167,9 +184,29 @@ struct DivBy<double> {
   }
   __device__ double first() const { return quot(a0); }
   __device__ double operator()(double a) const {
-    bool scale;
-    if (__builtin_amdgcn_div_scale(a, b, false, &scale) == ds) return quot(a);
+    if (scaled(a) == ds) return quot(a);
     return a / b;
+  }
+  // the same with the short way for zeros too (one more compare)
+  __device__ double maybe_zero(double a) const {
+    const double s = scaled(a);
+    if (s == ds || s != s) return quot(a);
+    return a / b;
+  }
+  // All of N quotients after DivBy(b), one test for the lot (equal or unordered: with ds NaN the
+  // divisor is zero or NaN, so every quotient is v_div_fixup's).
+  template <int N>
+  __device__ void all(const double a[N], double q[N]) const {
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < N; ++k) ok = ok && !__builtin_islessgreater(scaled(a[k]), ds);
+    if (ok) {
+#pragma unroll
+      for (int k = 0; k < N; ++k) q[k] = quot(a[k]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < N; ++k) q[k] = a[k] / b;
+    }
   }
 };
 #endif
@@ -185,6 +222,7 @@ struct KParams {
   int wb;             // well_balanced_flux_at_y_bc
   int bctc_ymin, bctc_ymax;
   int divx, divy;     // markstein_div mode of the divisions by dx and by dy (div_mode)
+  int divg;           // and by gm1
   long long plane;    // elements per field plane (pitch * Ny)
   double gamma0, gm1, entho;
   double dx, dy, inv_dx, inv_dy;  // inv_* = 1.0 / d (Viscosity.h:57-58), also RN(1/d) for markstein_div
@@ -192,6 +230,8 @@ struct KParams {
   double gdx_x, gdx_y;            // gx*dx, gy*dy (Update.h:131, for FSLP)
   double fslp_K;
   double kappa, mu;
+  double kf;                      // face conductivity 0.5 * (kappa + kappa) (ThermalConduction.h:62-65)
+  double qdx, qdy;                // 0.25 * inv_dx, 0.25 * inv_dy (Viscosity.h:62-106)
   double bctc_ymin_value, bctc_ymax_value;
   double eps_reset;               // misc.epsilon_reset_negative
   double inv_tc, inv_visc;        // parabolic inverse dts (constant over the grid)
@@ -200,33 +240,40 @@ struct KParams {
 
 // ------------------------------------------------------------------ state algebra
 
-// primToCons (States.h:19-30)
+// primToCons (States.h:19-30), given pg = p / (gamma - 1)
 template <typename R>
-FV2D_HD St<R> prim_to_cons(const St<R> &q, R gm1) {
+FV2D_HD St<R> prim_to_cons_pg(const St<R> &q, R pg) {
   typedef Ops<R> O;
   St<R> r;
   r.v[IR] = q.v[IR];
   r.v[IU] = q.v[IR] * q.v[IU];
   r.v[IV] = q.v[IR] * q.v[IV];
   R Ek = O::div(R(0.5) * (r.v[IU] * r.v[IU] + r.v[IV] * r.v[IV]), q.v[IR]);
-  r.v[IE] = Ek + O::div(q.v[IP], gm1);
+  r.v[IE] = Ek + pg;
   return r;
 }
+template <typename R>
+FV2D_HD St<R> prim_to_cons(const St<R> &q, R gm1) {
+  return prim_to_cons_pg(q, Ops<R>::div(q.v[IP], gm1));
+}
 
-// consToPrim (States.h:32-43)
+// consToPrim (States.h:32-43); byr: division by u's density (DivBy(u.v[IR])).
 template <typename R>
 FV2D_HD St<R> cons_to_prim(const St<R> &u, R gm1, const DivBy<R> &byr) {
   St<R> r;
   r.v[IR] = u.v[IR];
-  r.v[IU] = byr.first();
-  r.v[IV] = byr(u.v[IV]);
+  const R m[2] = {u.v[IU], u.v[IV]};
+  R w[2];
+  byr.template all<2>(m, w);
+  r.v[IU] = w[0];
+  r.v[IV] = w[1];
   R Ek = R(0.5) * r.v[IR] * (r.v[IU] * r.v[IU] + r.v[IV] * r.v[IV]);
   r.v[IP] = (u.v[IE] - Ek) * gm1;
   return r;
 }
 template <typename R>
 FV2D_HD St<R> cons_to_prim(const St<R> &u, R gm1) {
-  return cons_to_prim(u, gm1, DivBy<R>(u.v[IR], u.v[IU]));
+  return cons_to_prim(u, gm1, DivBy<R>(u.v[IR]));
 }
 
 // Negative density / pressure clamp of checkNegatives (SimInfo.h:617-626), on one cell.
@@ -282,20 +329,22 @@ FV2D_HD R plm_face(R q, R slope, R sign) {
 // All take primitive face states in the sweep frame (u normal) and return the flux in
 // that frame plus the interface pressure pout.
 
-// hll (RiemannSolvers.h:6-51), Davis wave-speed estimates
+// hll (RiemannSolvers.h:6-51), Davis wave-speed estimates. p / (gamma - 1) is a division by a
+// constant (entho = RN(1 / gm1), divg its mode, see markstein_div).
 template <typename R>
-FV2D_HD void hll(const St<R> &qL, const St<R> &qR, R gamma0, R gm1, St<R> &flux, R &pout) {
+FV2D_HD void hll(const St<R> &qL, const St<R> &qR, R gamma0, R gm1, R entho, int divg, St<R> &flux, R &pout) {
   typedef Ops<R> O;
   const R aL = speed_of_sound(qL, gamma0);
   const R aR = speed_of_sound(qR, gamma0);
   const R SL = O::min_(qL.v[IU] - aL, qR.v[IU] - aR);
   const R SR = O::max_(qL.v[IU] + aL, qR.v[IU] + aR);
 
+  const R pgL = O::div_c(qL.v[IP], gm1, entho, divg), pgR = O::div_c(qR.v[IP], gm1, entho, divg);
   // physical flux (RiemannSolvers.h:21-29)
   St<R> FL, FR;
   {
     const R Ek = R(0.5) * qL.v[IR] * (qL.v[IU] * qL.v[IU] + qL.v[IV] * qL.v[IV]);
-    const R E = O::div(qL.v[IP], gm1) + Ek;
+    const R E = pgL + Ek;
     FL.v[0] = qL.v[IR] * qL.v[IU];
     FL.v[1] = qL.v[IR] * qL.v[IU] * qL.v[IU] + qL.v[IP];
     FL.v[2] = qL.v[IR] * qL.v[IU] * qL.v[IV];
@@ -303,7 +352,7 @@ FV2D_HD void hll(const St<R> &qL, const St<R> &qR, R gamma0, R gm1, St<R> &flux,
   }
   {
     const R Ek = R(0.5) * qR.v[IR] * (qR.v[IU] * qR.v[IU] + qR.v[IV] * qR.v[IV]);
-    const R E = O::div(qR.v[IP], gm1) + Ek;
+    const R E = pgR + Ek;
     FR.v[0] = qR.v[IR] * qR.v[IU];
     FR.v[1] = qR.v[IR] * qR.v[IU] * qR.v[IU] + qR.v[IP];
     FR.v[2] = qR.v[IR] * qR.v[IU] * qR.v[IV];
@@ -318,18 +367,15 @@ FV2D_HD void hll(const St<R> &qL, const St<R> &qR, R gamma0, R gm1, St<R> &flux,
     pout = qR.v[IP];
   } else {
     // (SR*FL - SL*FR + SL*SR*(uR - uL)) / (SR - SL), uL/uR from primToCons
-    const St<R> uL = prim_to_cons(qL, gm1);
-    const St<R> uR = prim_to_cons(qR, gm1);
+    const St<R> uL = prim_to_cons_pg(qL, pgL);
+    const St<R> uR = prim_to_cons_pg(qR, pgR);
     pout = R(0.5) * (qL.v[IP] + qR.v[IP]);
     const R SLSR = SL * SR;
     const R den = SR - SL;
     R num[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) num[k] = FL.v[k] * SR - FR.v[k] * SL + (uR.v[k] - uL.v[k]) * SLSR;
-    const DivBy<R> byd(den, num[0]);
-    flux.v[0] = byd.first();
-#pragma unroll
-    for (int k = 1; k < 4; ++k) flux.v[k] = byd(num[k]);
+    DivBy<R>(den).template all<4>(num, flux.v);
   }
 }
 
@@ -345,10 +391,11 @@ FV2D_HD void hllc(const St<R> &qL, const St<R> &qR, R gamma0, R entho, St<R> &fl
   const R rL = qL.v[IR], uL = qL.v[IU], vL = qL.v[IV], pL = qL.v[IP];
   const R rR = qR.v[IR], uR = qR.v[IU], vR = qR.v[IV], pR = qR.v[IP];
 
-  const R cfastL = speed_of_sound(qL, gamma0);
-  const R cfastR = speed_of_sound(qR, gamma0);
-
-  const R cmax = O::max_(cfastL, cfastR);
+  // max(cfastL, cfastR) of the two speeds of sound (States.h:45-46) with one square root: a
+  // correctly rounded square root is monotone, so sqrt(max) is the larger root bit for bit; a
+  // negative or NaN argument loses against the other one in both forms, and two of them give NaN.
+  // (FP32 form: v_sqrt_f32 is monotone too, checked over all floats.)
+  const R cmax = O::sqrt_(O::max_(O::div(pL * gamma0, rL), O::div(pR * gamma0, rR)));
   const R SL = O::min_(uL, uR) - cmax;
   const R SR = O::max_(uL, uR) + cmax;
 
@@ -356,9 +403,9 @@ FV2D_HD void hllc(const St<R> &qL, const St<R> &qR, R gamma0, R entho, St<R> &fl
   const R rcR = rR * (SR - uR);
 
   const R den = rcR + rcL;
-  const DivBy<R> byd(den, rcR * uR + rcL * uL + (pL - pR));
-  const R uS = byd.first();
-  const R pS = byd(rcR * pL + rcL * pR + rcL * rcR * (uL - uR));
+  const DivBy<R> byd(den, rcR * pL + rcL * pR + rcL * rcR * (uL - uR));
+  const R pS = byd.first();
+  const R uS = byd.maybe_zero(rcR * uR + rcL * uL + (pL - pR));  // zero between equal states at rest
 
   // branches SL > 0 (left state), uS > 0 (left star), SR > 0 (right star), else (right state)
   const bool left = (SL > R(0)) || (uS > R(0));
@@ -393,7 +440,8 @@ FV2D_HD void hllc(const St<R> &qL, const St<R> &qR, R gamma0, R entho, St<R> &fl
 
 // fslp (RiemannSolvers.h:137-171); Kokkos::max/min are (a < b ? b : a) / (b < a ? b : a).
 template <typename R>
-FV2D_HD void fslp(const St<R> &qL, const St<R> &qR, R gamma0, R gm1, R K, R gdx, St<R> &flux, R &pout) {
+FV2D_HD void fslp(const St<R> &qL, const St<R> &qR, R gamma0, R gm1, R entho, int divg, R K, R gdx, St<R> &flux,
+                  R &pout) {
   typedef Ops<R> O;
   const R rhoL = qL.v[IR], uL = qL.v[IU], pL = qL.v[IP];
   const R csL = O::sqrt_(O::div(gamma0 * pL, rhoL));
@@ -415,7 +463,7 @@ FV2D_HD void fslp(const St<R> &qL, const St<R> &qR, R gamma0, R gm1, R K, R gdx,
   const R sv = up ? qL.v[IV] : qR.v[IV];
   const R sp = up ? qL.v[IP] : qR.v[IP];
   const R Ekstar = R(0.5) * sr * (su * su + sv * sv);
-  const R Estar = Ekstar + O::div(sp, gm1);
+  const R Estar = Ekstar + O::div_c(sp, gm1, entho, divg);
 
   flux.v[IR] = ustar * sr;
   flux.v[IU] = ustar * sr * su + Pi;
@@ -425,12 +473,12 @@ FV2D_HD void fslp(const St<R> &qL, const St<R> &qR, R gamma0, R gm1, R K, R gdx,
 }
 
 template <int RIEM, typename R>
-FV2D_HD void riemann(const St<R> &qL, const St<R> &qR, R gamma0, R gm1, R entho, R K, R gdx, St<R> &flux,
+FV2D_HD void riemann(const St<R> &qL, const St<R> &qR, R gamma0, R gm1, R entho, int divg, R K, R gdx, St<R> &flux,
                      R &pout) {
   if (RIEM == HLL)
-    hll(qL, qR, gamma0, gm1, flux, pout);
+    hll(qL, qR, gamma0, gm1, entho, divg, flux, pout);
   else if (RIEM == FSLP)
-    fslp(qL, qR, gamma0, gm1, K, gdx, flux, pout);
+    fslp(qL, qR, gamma0, gm1, entho, divg, K, gdx, flux, pout);
   else
     hllc(qL, qR, gamma0, entho, flux, pout);
 }

@@ -41,6 +41,7 @@ constexpr size_t NA_STATE_BYTES = 4 * sizeof(double) * (size_t)FV2D_NOALLOC_MAX_
 constexpr size_t NA_BYTES = NA_STATE + 3 * NA_STATE_BYTES;
 static_assert(NA_DTS % 256 == 0 && NA_GRAV % 256 == 0 && NA_STATE % 256 == 0, "scratch regions must stay aligned");
 static_assert(sizeof(StepCtl) <= NA_PARTS, "control block region too small");
+static_assert(ACC_WORDS <= FV2D_NOALLOC_MAX_WORKGROUPS, "the dt slots share the partials' region");
 
 }  // namespace
 
@@ -106,8 +107,7 @@ int fv2d_run_noalloc(const fv2d_params *p, const double *q_in, double *q_out, do
   SimDev d;
   d.p = *p;
   build_kparams(p, pitch, d.kp);
-  d.geom = sim_geom(p);
-  d.nparts = d.geom.nblocks;
+  sim_set_geom(d);
   if (d.nparts > FV2D_NOALLOC_MAX_WORKGROUPS)
     return fail(FV2D_E_INVALID, "fv2d_run_noalloc: %d workgroups exceed the partials capacity %d (raise seg_rows)",
                 d.nparts, FV2D_NOALLOC_MAX_WORKGROUPS);
@@ -158,7 +158,7 @@ int fv2d_run_noalloc(const fv2d_params *p, const double *q_in, double *q_out, do
     hipLaunchKernelGGL(init_state_kernel<double>, dim3(grid_1d(n)), dim3(AUX_THREADS), 0, d.stream, d.kp, q_in,
                        (double *)d.U, (double *)d.Q0);
   NA_HIP(hipGetLastError());
-  hipLaunchKernelGGL(clear_ctl_kernel, dim3(1), dim3(1), 0, d.stream, d.ctl);
+  hipLaunchKernelGGL(clear_ctl_kernel, dim3(1), dim3(64), 0, d.stream, d.ctl, sim_acc(d));
   NA_HIP(hipGetLastError());
   NA_HIP(sim_launch_dt_tiles(d, d.Q0, 1));
   NA_HIP(sim_launch_reduce(d, 0, nullptr));

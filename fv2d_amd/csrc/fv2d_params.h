@@ -9,7 +9,7 @@
 #include <string>
 
 #include "../../include/fv2d_amd.h"
-#include "fv2d_stage.h"
+#include "fv2d_march.h"
 
 namespace fv2d {
 
@@ -94,6 +94,7 @@ inline void build_kparams(const fv2d_params *p, int pitch, KParams &kp) {
   kp.inv_dy = 1.0 / kp.dy;
   kp.divx = div_mode(kp.dx);
   kp.divy = div_mode(kp.dy);
+  kp.divg = div_mode(kp.gm1);
   kp.gxf = (double)(float)p->gx;
   kp.gyf = (double)(float)p->gy;
   kp.gdx_x = p->gx * kp.dx;
@@ -101,6 +102,9 @@ inline void build_kparams(const fv2d_params *p, int pitch, KParams &kp) {
   kp.fslp_K = p->fslp_K;
   kp.kappa = p->kappa;
   kp.mu = p->mu;
+  kp.kf = 0.5 * (p->kappa + p->kappa);
+  kp.qdx = 0.25 * kp.inv_dx;
+  kp.qdy = 0.25 * kp.inv_dy;
   kp.bctc_ymin_value = p->bctc_ymin_value;
   kp.bctc_ymax_value = p->bctc_ymax_value;
   kp.eps_reset = p->epsilon_reset_negative;
@@ -138,6 +142,46 @@ inline int pick_seg_rows(const fv2d_params *p, int nw) {
   const long long strips = (p->Nx + 61) / 62;
   while (seg > step && strips * ((p->Ny + seg - 1) / seg) < 2048) seg -= step;
   return seg;
+}
+
+// Rows per task of the march kernel. A SIMD that holds w waves of S rows each is busy for about
+// (S + p) * sqrt(L^2 + (w I)^2): p rows' worth of work and latency before the first row, L the
+// dependency chain of a row, I its VALU time (fitted at KH: p = 0.95; FP64 L = 2.3 us, I = 1.5 us,
+// FP32 1.1, 0.55; measured per row at w = 1..4: FP64 2.6, 3.4, 4.7, 6.4, FP32 1.2, 1.5, 1.9, 2.3).
+// S is the one of least time over w = 1 .. the resident waves, then whole rounds of those, so that
+// every SIMD finishes together: at KH 2048^2 FP64 (S, us per step) 18: 235, 16 (9% into a second
+// round): 249. At most 40 rows, since the waves of one long round drift apart (KH 4096^2: one
+// round of 70 rows 930, two of 35 915).
+inline int pick_march_rows(const fv2d_params *p) {
+  const bool f64 = p->precision == FV2D_FP64;
+  const bool xg = p->gravity_mode || p->well_balanced_flux_at_y_bc || p->bctc_ymin || p->bctc_ymax;
+  const int simds = 1024, slots = march_wpe(f64, xg && (p->tc_active || p->visc_active));
+  const double P = 0.95, L = f64 ? 2.3 : 1.1, I = f64 ? 1.5 : 0.55;
+  const long long nsx = (p->Nx + MARCH_OUT - 1) / MARCH_OUT;
+  int best = 40;
+  double best_t = 1e300;
+  for (int k = 1;; ++k) {
+    const int w = k <= slots ? k : slots, rounds = k <= slots ? 1 : k - slots + 1;
+    const long long nsy = (long long)simds * w * rounds / nsx;
+    if (nsy < 1) continue;
+    const int S = (int)((p->Ny + nsy - 1) / nsy);
+    const double t = (S + P) * rounds * sqrt(L * L + w * w * I * I);
+    if (S <= 40 && t < best_t) {
+      best = S;
+      best_t = t;
+    }
+    if (S == 1 || (S <= 20 && k >= slots)) return best;
+  }
+}
+
+// Work split of the march kernel, the single-grid kernel unless chunk_rows asks for the strip
+// kernel (ntasks = 0). The FP32 form on an FP64 state also takes the strip kernel: it is held by
+// memory traffic, and the march, which reads U of a row again at its update, takes 680 us per step
+// at KH 4096^2 against 627.
+inline MarchGeom sim_march_geom(const fv2d_params *p) {
+  MarchGeom g = {0, 0, 0, 0};
+  if (p->chunk_rows > 0 || p->precision == FV2D_FP32_STATE64) return g;
+  return march_geom(p->Nx, p->Ny, p->seg_rows > 0 ? p->seg_rows : pick_march_rows(p));
 }
 
 // Strip geometry of the single-grid kernel: the banded long-then-short schedule when the

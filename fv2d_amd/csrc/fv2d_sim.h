@@ -10,6 +10,8 @@
 #include "../../include/fv2d_amd.h"
 #include "fv2d_aux.h"
 #include "fv2d_device.h"
+#include "fv2d_march_device.h"
+#include "fv2d_params.h"
 
 namespace fv2d {
 
@@ -17,7 +19,8 @@ namespace fv2d {
 struct SimDev {
   fv2d_params p;
   KParams kp;
-  StripGeom geom;
+  StripGeom geom;   // strip kernel (explicit chunk_rows)
+  MarchGeom march;  // march kernel (ntasks = 0: the strip kernel runs)
   int nparts = 0;  // per-workgroup partial maxima of the dt reduction (= geom.nblocks)
   hipStream_t stream = nullptr;
   void *U = nullptr, *Us = nullptr, *Q0 = nullptr;  // SoA planes, row pitch kp.pitch
@@ -30,6 +33,22 @@ struct SimDev {
   void *mark_ctx = nullptr;
 };
 
+// The stage kernel and work split of the parameters.
+inline void sim_set_geom(SimDev &d) {
+  d.geom = sim_geom(&d.p);
+  d.march = sim_march_geom(&d.p);
+  d.nparts = d.geom.nblocks;
+}
+
+// The march kernel's slots share the buffer of the strip kernel's partials (sim_partials_bytes).
+inline unsigned long long *sim_acc(const SimDev &d) {
+  return d.march.ntasks ? (unsigned long long *)d.partials : nullptr;
+}
+inline size_t sim_partials_bytes(const SimDev &d) {
+  const size_t n = d.march.ntasks && d.nparts < ACC_WORDS ? ACC_WORDS : d.nparts;
+  return n * sizeof(double);
+}
+
 // Sets the message fv2d_last_error(NULL) returns (fv2d_capi.hip).
 void set_global_error(const char *msg);
 
@@ -41,27 +60,33 @@ inline bool sim_fp32s64(const SimDev &d) { return d.p.precision == FV2D_FP32_STA
 // Max hyperbolic inverse dt of Q0 (from_q0) or of reset(consToPrim(src)) into the partials.
 inline hipError_t sim_launch_dt_tiles(SimDev &d, const void *src, int from_q0) {
   const dim3 grid(d.nparts);
+  unsigned long long *acc = sim_acc(d);
   if (sim_fp32(d))
     hipLaunchKernelGGL((dt_cells_kernel<float, float>), grid, dim3(256), 0, d.stream, d.kp, (const float *)src, from_q0,
-                       d.partials, d.nparts);
+                       d.partials, d.nparts, acc);
   else if (sim_fp32s64(d))
     hipLaunchKernelGGL((dt_cells_kernel<float, double>), grid, dim3(256), 0, d.stream, d.kp, (const double *)src,
-                       from_q0, d.partials, d.nparts);
+                       from_q0, d.partials, d.nparts, acc);
   else
     hipLaunchKernelGGL((dt_cells_kernel<double, double>), grid, dim3(256), 0, d.stream, d.kp, (const double *)src,
-                       from_q0, d.partials, d.nparts);
+                       from_q0, d.partials, d.nparts, acc);
   return hipGetLastError();
 }
 
 inline hipError_t sim_launch_reduce(SimDev &d, int advance, double *dts_log) {
-  hipLaunchKernelGGL(reduce_kernel, dim3(1), dim3(1024), 0, d.stream, d.ctl, d.partials, d.nparts, d.kp, advance,
-                     dts_log);
+  if (d.march.ntasks)
+    hipLaunchKernelGGL(reduce_acc_kernel, dim3(1), dim3(64), 0, d.stream, d.ctl, sim_acc(d), d.kp, advance, dts_log);
+  else
+    hipLaunchKernelGGL(reduce_kernel, dim3(1), dim3(1024), 0, d.stream, d.ctl, d.partials, d.nparts, d.kp, advance,
+                       dts_log);
   return hipGetLastError();
 }
 
 // One stage: out = [avg +] src + dt L(Q(src or Q0)).
 inline hipError_t sim_launch_stage(SimDev &d, const void *src, int qsrc, const void *avg, void *out, int epilogue) {
   const int recon = (d.p.reconstruction == FV2D_PLM) ? PLM : PCM;
+  const bool tc = d.p.tc_active != 0, visc = d.p.visc_active != 0;
+  const StageClass cls = {recon, d.p.riemann_solver, tc, visc, needs_xg(d.kp), 0};
   hipError_t e;
   if (d.mark && (e = d.mark(d.mark_ctx)) != hipSuccess) return e;
   if (sim_fp32(d)) {
@@ -73,10 +98,11 @@ inline hipError_t sim_launch_stage(SimDev &d, const void *src, int qsrc, const v
     io.grav_row = d.grav_row;
     io.ctl = d.ctl;
     io.partials = d.partials;
+    io.acc = sim_acc(d);
     io.qsrc = qsrc;
     io.epilogue = epilogue;
-    e = launch_stage_fp32(d.kp, io, d.geom, recon, d.p.riemann_solver, d.p.tc_active != 0, d.p.visc_active != 0,
-                          d.stream);
+    e = d.march.ntasks ? launch_march_fp32(cls, d.kp, io, d.march, d.stream)
+                       : launch_stage_fp32(d.kp, io, d.geom, recon, d.p.riemann_solver, tc, visc, d.stream);
   } else {
     StageIO<double> io;
     io.src = (const double *)src;
@@ -86,14 +112,14 @@ inline hipError_t sim_launch_stage(SimDev &d, const void *src, int qsrc, const v
     io.grav_row = d.grav_row;
     io.ctl = d.ctl;
     io.partials = d.partials;
+    io.acc = sim_acc(d);
     io.qsrc = qsrc;
     io.epilogue = epilogue;
     if (sim_fp32s64(d))
-      e = launch_stage_fp32s64(d.kp, io, d.geom, recon, d.p.riemann_solver, d.p.tc_active != 0,
-                               d.p.visc_active != 0, d.stream);
+      e = launch_stage_fp32s64(d.kp, io, d.geom, recon, d.p.riemann_solver, tc, visc, d.stream);
     else
-      e = launch_stage_fp64(d.kp, io, d.geom, recon, d.p.riemann_solver, d.p.tc_active != 0,
-                            d.p.visc_active != 0, d.stream);
+      e = d.march.ntasks ? launch_march_fp64(cls, d.kp, io, d.march, d.stream)
+                         : launch_stage_fp64(d.kp, io, d.geom, recon, d.p.riemann_solver, tc, visc, d.stream);
   }
   if (e != hipSuccess) return e;
   if (d.mark && (e = d.mark(d.mark_ctx)) != hipSuccess) return e;

@@ -45,6 +45,14 @@ struct StepCtl {
   unsigned long long neg_rho, neg_prs, nan_cnt;  // running totals of the reset
 };
 
+// The march kernel's dt reduction: its waves (task t) take part in the integer maximum of slot
+// t % ACC_SLOTS, on the bits of the inverse dt (which order non-negative doubles, so the result
+// does not depend on the order of the waves). The slots lie in cache lines of their own: with one
+// slot for all, the waves of a launch, which end together, queue at it for about 8 ns each (FP32
+// Sedov 1024^2: 75 us per step against 40).
+constexpr int ACC_SLOTS = 64, ACC_STRIDE = 16;  // stride in 8-byte words
+constexpr int ACC_WORDS = ACC_SLOTS * ACC_STRIDE;
+
 enum : int { QSRC_U_RESET = 0, QSRC_U = 1, QSRC_Q0 = 2 };
 
 template <typename S>
@@ -55,7 +63,8 @@ struct StageIO {
   S *out;                 // output U planes
   const float *grav_row;  // analytical gravity per row (Ny), else null
   StepCtl *ctl;
-  double *partials;       // per-workgroup max inverse dt (epilogue)
+  double *partials;       // per-workgroup max inverse dt (epilogue, strip kernel)
+  unsigned long long *acc;  // ACC_SLOTS running maxima (epilogue, march kernel)
   int qsrc;               // QSRC_*
   int epilogue;
 };
@@ -64,13 +73,15 @@ struct StageIO {
 // precision; buffers are typed by it.
 struct BatchJob {
   KParams kp;
-  int nblocks;   // workgroup items of this job (strip geometry)
+  int nblocks;   // workgroup items of this job (strip geometry), or wave tasks (march)
   int seg;       // rows per segment
   int nsx, nsy;
+  int march;     // the class runs the march kernel
   void *U, *Us, *Q0;
   const float *grav_row;
   StepCtl *ctl;
   double *partials;
+  unsigned long long *acc;
   int rk2;       // SSP-RK2 (else Euler)
   int used;      // slot holds a job
   int cls;       // kernel class (index into the batch's class table)
@@ -255,17 +266,171 @@ struct LaneRegs {
   double inv;
 };
 
-// XG: gravity, the well-balanced wall flux or wall conduction modes are on; without it
-// their code is compiled out.
-// NW_: rows per chunk = waves per workgroup (a chunk_rows_supported value).
-// DIVF_: how the update phases divide by dx and dy (FP64): DIVF_RUNTIME picks the exact-multiply
+// Per-cell pieces of the stage shared by its two kernels (StripStage below, MarchStage in
+// fv2d_march.h): loads with the boundary rules, primitives, the update's accumulation and the
+// end of the update (RK2 average, store, the next step's dt term).
+//
+// DIVF: how the update phases divide by dx and dy (FP64): DIVF_RUNTIME picks the exact-multiply
 // or the general form per call from kp (emulation, batch kernels, FP32 form); the single-grid
 // FP64 kernels are built once with DIVF_EXACT (both cell sizes powers of two) and once with
 // DIVF_GENERAL, so each holds only the form it runs.
 enum : int { DIVF_RUNTIME = 0, DIVF_EXACT = 1, DIVF_GENERAL = 2 };
+template <typename R, typename S, bool TC, int DIVF>
+struct StageOps {
+  // Storage values of domain-relative cell (gi, gj), ghosts included (mapped to their source
+  // cell; fx / fy: the normal velocity changes sign). UNI: gj is the same for the whole wave.
+  template <bool UNI>
+  static FV2D_HD void fetch_raw(int gi, int gj, const KParams &kp, const StageIO<S> &io, S raw[4], bool &fx,
+                                bool &fy) {
+    fx = false;
+    fy = false;
+    const int si = (gi >= 0 && gi < kp.Nx) ? gi : map_ghost(gi, kp.Nx, kp.bcx, fx);
+    const int sj = (gj >= 0 && gj < kp.Ny) ? gj : map_ghost(gj, kp.Ny, kp.bcy, fy);
+    const S *base = (io.qsrc == QSRC_Q0) ? io.q0 : io.src;
+    if (UNI) {
+      const S *row = base + (long long)sj * kp.pitch;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) raw[v] = URow<S>(row + (long long)v * kp.plane)[si];
+    } else {
+      const long long k = (long long)sj * kp.pitch + si;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) raw[v] = base[v * kp.plane + k];
+    }
+  }
+
+  // Primitives from storage values: Q0 as given, else consToPrim (+ reset); with conduction
+  // also T = p / rho (ThermalConduction.h:56-60), which shares consToPrim's divisor rho
+  // unless the reset changed it.
+  static FV2D_HD void raw_to_q(const S raw[4], bool fx, bool fy, const KParams &kp, const StageIO<S> &io,
+                               St<R> &q, R &t) {
+    if (io.qsrc == QSRC_Q0) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) q.v[v] = R(raw[v]);
+      if (TC) t = Ops<R>::div(q.v[IP], q.v[IR]);
+    } else {
+      St<R> u;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) u.v[v] = R(raw[v]);
+      const DivBy<R> byr(u.v[IR]);
+      q = cons_to_prim(u, R(kp.gm1), byr);
+      if (io.qsrc == QSRC_U_RESET) reset_negative(q, R(kp.eps_reset));
+      if (TC) {
+        if (q.v[IR] == u.v[IR])
+          t = byr(q.v[IP]);
+        else
+          t = Ops<R>::div(q.v[IP], q.v[IR]);
+      }
+    }
+    if (fx) q.v[IU] = -q.v[IU];
+    if (fy) q.v[IV] = -q.v[IV];
+  }
+
+  // Both cell sizes are powers of two (the FP64 divisions by dx and dy are exact multiplies):
+  // the update phases are then compiled with that mode fixed, which drops the mode tests of
+  // every division from the chunk loop. The FP32 form multiplies in every mode.
+  static FV2D_HD bool exact_dxdy(const KParams &kp) {
+    if (DIVF != DIVF_RUNTIME) return DIVF == DIVF_EXACT;
+    return sizeof(R) == 8 && kp.divx == DIV_EXACT && kp.divy == DIV_EXACT;
+  }
+
+  // Accumulator of the update. FP64: U itself, every term added in the reference's order
+  // (Update.h:158-166, States.h:49-101). FP32 form: the increment dt*dF of the step in
+  // FP32, added to U once at the end (in FP32 for the FP32 state, in FP64 for the FP64 one).
+  typedef typename std::conditional<sizeof(R) == 8, double, float>::type A;
+
+  // U += ((FL - FR) * dt) / d (Update.h:158-159); FP32 form: (FL - FR) * (dt / d).
+  static FV2D_HD void add_flux(A acc[4], const R FL[4], const R FR[4], double dt, double dt_d, double d, double rd,
+                               int mode) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      if (sizeof(R) == 8)
+        acc[v] = acc[v] + A(Ops<double>::div_c((double)(FL[v] - FR[v]) * dt, d, rd, mode));
+      else
+        acc[v] = acc[v] + A(FL[v] - FR[v]) * A(dt_d);
+    }
+  }
+
+  // Gravity source (Update.h:161-166): always into the y momentum; energy from the mass
+  // fluxes of the sweep.
+  static FV2D_HD void add_gravity(A acc[4], R rho, R FL0, R FR0, double dt, double g) {
+    acc[IV] = acc[IV] + A(dt) * A(rho) * A(g);
+    acc[IE] = acc[IE] + A(dt) * A(0.5) * (A(FL0) + A(FR0)) * A(g);
+  }
+
+  // End of the update of cell (gi, j): U + increment, the RK2 average, the store and the epilogue.
+  static FV2D_HD void finish_cell(int gi, int j, const A acc[4], const S u[4], const S u0[4], const KParams &kp,
+                                  const StageIO<S> &io, int divx, int divy, unsigned &neg_rho, unsigned &neg_prs,
+                                  unsigned &nan_cnt, double &inv_max) {
+    S uns[4];
+    if (sizeof(R) == 8 || sizeof(S) == 8) {
+      double un64[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) un64[v] = (sizeof(R) == 8) ? double(acc[v]) : double(u[v]) + double(acc[v]);
+      // SSP-RK2 average (Update.h:214-220)
+      if (io.avg) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) un64[v] = 0.5 * (double(u0[v]) + un64[v]);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) uns[v] = S(un64[v]);
+    } else {
+      // FP32 state: U + dt*dF and the RK2 average in FP32, each rounded once, like the storage
+#pragma unroll
+      for (int v = 0; v < 4; ++v) uns[v] = S(u[v] + S(acc[v]));
+      if (io.avg) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) uns[v] = S(0.5f) * (u0[v] + uns[v]);
+      }
+    }
+
+    const long long k = (long long)j * kp.pitch;
+    St<R> un;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      URow<S>(io.out + (k + (long long)v * kp.plane)).store(gi, uns[v]);
+      un.v[v] = R(uns[v]);
+    }
+
+    // epilogue: consToPrim + checkNegatives (SimInfo.h:576-646) and the next dt's cell term
+    if (io.epilogue) {
+      const DivBy<R> byr(un.v[IR]);
+      St<R> q = cons_to_prim(un, R(kp.gm1), byr);
+      const R eps = R(kp.eps_reset);
+      if (q.v[IR] < R(0)) {
+        q.v[IR] = eps;
+        neg_rho += 1;
+      }
+      if (q.v[IP] < R(0)) {
+        q.v[IP] = eps;
+        neg_prs += 1;
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) nan_cnt += (q.v[v] != q.v[v]) ? 1u : 0u;
+      // speedOfSound (States.h:45-46): (p * gamma) / rho, by the same divisor unless reset
+      R c2;
+      if (q.v[IR] == un.v[IR])
+        c2 = byr(q.v[IP] * R(kp.gamma0));
+      else
+        c2 = Ops<R>::div(q.v[IP] * R(kp.gamma0), q.v[IR]);
+      const double inv = inv_dt_hyp_cs(q, Ops<R>::sqrt_(c2), kp, divx, divy);
+      if (inv > inv_max) inv_max = inv;  // NaN never wins: the reference's fmax-based Max ignores it
+    }
+  }
+};
+
+// XG: gravity, the well-balanced wall flux or wall conduction modes are on; without it
+// their code is compiled out.
+// NW_: rows per chunk = waves per workgroup (a chunk_rows_supported value).
+// DIVF_: see StageOps.
 template <typename R, typename S, int RECON, int RIEM, bool TC, bool VISC, bool XG, int NW_,
           int DIVF_ = DIVF_RUNTIME>
-struct StripStage {
+struct StripStage : StageOps<R, S, TC, DIVF_> {
+  typedef StageOps<R, S, TC, DIVF_> Ops_;
+  using typename Ops_::A;
+  using Ops_::add_flux;
+  using Ops_::add_gravity;
+  using Ops_::exact_dxdy;
+  using Ops_::raw_to_q;
   static constexpr int NW = NW_;
   static constexpr int DIVF = DIVF_;
   static constexpr int NT = 64 * NW;
@@ -308,60 +473,12 @@ struct StripStage {
   static FV2D_HD int yslot(int j, int jb) { return (j - jb + 1) % NY; }
   static FV2D_HD int vslot(int j, int jb) { return (j - jb + 1) % NV; }
 
-  // Storage values of domain-relative cell (gi, gj), ghosts included (mapped to their source
-  // cell; fx / fy: the normal velocity changes sign). UNI: gj is the same for the whole wave.
-  template <bool UNI>
-  static FV2D_HD void fetch_raw(int gi, int gj, const KParams &kp, const StageIO<S> &io, S raw[4], bool &fx,
-                                bool &fy) {
-    fx = false;
-    fy = false;
-    const int si = (gi >= 0 && gi < kp.Nx) ? gi : map_ghost(gi, kp.Nx, kp.bcx, fx);
-    const int sj = (gj >= 0 && gj < kp.Ny) ? gj : map_ghost(gj, kp.Ny, kp.bcy, fy);
-    const S *base = (io.qsrc == QSRC_Q0) ? io.q0 : io.src;
-    if (UNI) {
-      const S *row = base + (long long)sj * kp.pitch;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) raw[v] = URow<S>(row + (long long)v * kp.plane)[si];
-    } else {
-      const long long k = (long long)sj * kp.pitch + si;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) raw[v] = base[v * kp.plane + k];
-    }
-  }
-
-  // Primitives from storage values: Q0 as given, else consToPrim (+ reset); with conduction
-  // also T = p / rho (ThermalConduction.h:56-60), which shares consToPrim's divisor rho
-  // unless the reset changed it.
-  static FV2D_HD void raw_to_q(const S raw[4], bool fx, bool fy, const KParams &kp, const StageIO<S> &io,
-                               St<R> &q, R &t) {
-    if (io.qsrc == QSRC_Q0) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) q.v[v] = R(raw[v]);
-      if (TC) t = Ops<R>::div(q.v[IP], q.v[IR]);
-    } else {
-      St<R> u;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) u.v[v] = R(raw[v]);
-      const DivBy<R> byr(u.v[IR], u.v[IU]);
-      q = cons_to_prim(u, R(kp.gm1), byr);
-      if (io.qsrc == QSRC_U_RESET) reset_negative(q, R(kp.eps_reset));
-      if (TC) {
-        if (q.v[IR] == u.v[IR])
-          t = byr(q.v[IP]);
-        else
-          t = Ops<R>::div(q.v[IP], q.v[IR]);
-      }
-    }
-    if (fx) q.v[IU] = -q.v[IU];
-    if (fy) q.v[IV] = -q.v[IV];
-  }
-
   // Primitive state (and T) of domain-relative cell (gi, gj), ghosts included.
   template <bool UNI>
   static FV2D_HD void fetch_q(int gi, int gj, const KParams &kp, const StageIO<S> &io, St<R> &q, R &t) {
     S raw[4];
     bool fx, fy;
-    fetch_raw<UNI>(gi, gj, kp, io, raw, fx, fy);
+    Ops_::template fetch_raw<UNI>(gi, gj, kp, io, raw, fx, fy);
     raw_to_q(raw, fx, fy, kp, io, q, t);
   }
 
@@ -442,7 +559,7 @@ struct StripStage {
       b.v[v] = (RECON == PLM) ? plm_face(hi, shi[v], R(-1)) : hi;
     }
     St<R> fs;
-    riemann<RIEM>(swap_uv(a), swap_uv(b), R(kp.gamma0), R(kp.gm1), R(kp.entho), R(kp.fslp_K), R(kp.gdx_y), fs,
+    riemann<RIEM>(swap_uv(a), swap_uv(b), R(kp.gamma0), R(kp.gm1), R(kp.entho), kp.divg, R(kp.fslp_K), R(kp.gdx_y), fs,
                   pout);
     f = swap_uv(fs);
   }
@@ -516,10 +633,10 @@ struct StripStage {
   static FV2D_HD void chunk_prefetch(int lane, int w, int xwn, int i0, int jn, const KParams &kp,
                                      const StageIO<S> &io, RowPrefetch<S> &p) {
     bool fx, fy;
-    fetch_raw<true>(i0 - 2 + lane, jn + 2 + w, kp, io, p.row, fx, fy);
+    Ops_::template fetch_raw<true>(i0 - 2 + lane, jn + 2 + w, kp, io, p.row, fx, fy);
     p.flags = (fx ? 1 : 0) | (fy ? 2 : 0);
     if (kPFX && w == xwn && lane < 2 * NW) {
-      fetch_raw<false>(i0 - 2 + STRIP_W + (lane & 1), jn + 2 + (lane >> 1), kp, io, p.extra, fx, fy);
+      Ops_::template fetch_raw<false>(i0 - 2 + STRIP_W + (lane & 1), jn + 2 + (lane >> 1), kp, io, p.extra, fx, fy);
       p.flags |= (fx ? 4 : 0) | (fy ? 8 : 0);
     }
   }
@@ -566,7 +683,7 @@ struct StripStage {
     }
     St<R> f;
     R pout;
-    riemann<RIEM>(a, b, R(kp.gamma0), R(kp.gm1), R(kp.entho), R(kp.fslp_K), R(kp.gdx_x), f, pout);
+    riemann<RIEM>(a, b, R(kp.gamma0), R(kp.gm1), R(kp.entho), kp.divg, R(kp.fslp_K), R(kp.gdx_x), f, pout);
 #pragma unroll
     for (int v = 0; v < 4; ++v) r.fx[v] = f.v[v];
   }
@@ -586,14 +703,6 @@ struct StripStage {
     }
     if (XG && j == kp.Ny - 2) sm.pw[lane] = r.py;
     if (VISC) visc_yface(lane, j, jb, sm, kp);
-  }
-
-  // Both cell sizes are powers of two (the FP64 divisions by dx and dy are exact multiplies):
-  // the update phases are then compiled with that mode fixed, which drops the mode tests of
-  // every division from the chunk loop. The FP32 form multiplies in every mode.
-  static FV2D_HD bool exact_dxdy(const KParams &kp) {
-    if (DIVF != DIVF_RUNTIME) return DIVF == DIVF_EXACT;
-    return sizeof(R) == 8 && kp.divx == DIV_EXACT && kp.divy == DIV_EXACT;
   }
 
   // Update part 1: conduction and viscous terms of the x face (lane, lane+1) of row jc+w.
@@ -635,30 +744,6 @@ struct StripStage {
       r.vx[1] = mu * tau_xy;
       r.vx[2] = mu * (tau_xx * qiu + tau_xy * qiv);
     }
-  }
-
-  // Accumulator of the update. FP64: U itself, every term added in the reference's order
-  // (Update.h:158-166, States.h:49-101). FP32 form: the increment dt*dF of the step in
-  // FP32, added to U once at the end (in FP32 for the FP32 state, in FP64 for the FP64 one).
-  typedef typename std::conditional<sizeof(R) == 8, double, float>::type A;
-
-  // U += ((FL - FR) * dt) / d (Update.h:158-159); FP32 form: (FL - FR) * (dt / d).
-  static FV2D_HD void add_flux(A acc[4], const R FL[4], const R FR[4], double dt, double dt_d, double d, double rd,
-                               int mode) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      if (sizeof(R) == 8)
-        acc[v] = acc[v] + A(Ops<double>::div_c((double)(FL[v] - FR[v]) * dt, d, rd, mode));
-      else
-        acc[v] = acc[v] + A(FL[v] - FR[v]) * A(dt_d);
-    }
-  }
-
-  // Gravity source (Update.h:161-166): always into the y momentum; energy from the mass
-  // fluxes of the sweep.
-  static FV2D_HD void add_gravity(A acc[4], R rho, R FL0, R FR0, double dt, double g) {
-    acc[IV] = acc[IV] + A(dt) * A(rho) * A(g);
-    acc[IE] = acc[IE] + A(dt) * A(0.5) * (A(FL0) + A(FR0)) * A(g);
   }
 
   // Update part 2: the cell (lane, jc+w) (needs fxl, tcxl, vxl from lane-1).
@@ -780,60 +865,7 @@ struct StripStage {
       acc[IE] = acc[IE] + A(fxe + fye) * A(dt);
     }
 
-    S uns[4];
-    if (sizeof(R) == 8 || sizeof(S) == 8) {
-      double un64[4];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) un64[v] = (sizeof(R) == 8) ? double(acc[v]) : double(r.u[v]) + double(acc[v]);
-      // SSP-RK2 average (Update.h:214-220)
-      if (io.avg) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) un64[v] = 0.5 * (double(r.u0[v]) + un64[v]);
-      }
-#pragma unroll
-      for (int v = 0; v < 4; ++v) uns[v] = S(un64[v]);
-    } else {
-      // FP32 state: U + dt*dF and the RK2 average in FP32, each rounded once, like the storage
-#pragma unroll
-      for (int v = 0; v < 4; ++v) uns[v] = S(r.u[v] + S(acc[v]));
-      if (io.avg) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) uns[v] = S(0.5f) * (r.u0[v] + uns[v]);
-      }
-    }
-
-    const long long k = (long long)j * kp.pitch;
-    St<R> un;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      URow<S>(io.out + (k + (long long)v * kp.plane)).store(gi, uns[v]);
-      un.v[v] = R(uns[v]);
-    }
-
-    // epilogue: consToPrim + checkNegatives (SimInfo.h:576-646) and the next dt's cell term
-    if (io.epilogue) {
-      const DivBy<R> byr(un.v[IR], un.v[IU]);
-      St<R> q = cons_to_prim(un, R(kp.gm1), byr);
-      const R eps = R(kp.eps_reset);
-      if (q.v[IR] < R(0)) {
-        q.v[IR] = eps;
-        r.neg_rho += 1;
-      }
-      if (q.v[IP] < R(0)) {
-        q.v[IP] = eps;
-        r.neg_prs += 1;
-      }
-#pragma unroll
-      for (int v = 0; v < 4; ++v) r.nan_cnt += (q.v[v] != q.v[v]) ? 1u : 0u;
-      // speedOfSound (States.h:45-46): (p * gamma) / rho, by the same divisor unless reset
-      R c2;
-      if (q.v[IR] == un.v[IR])
-        c2 = byr(q.v[IP] * R(kp.gamma0));
-      else
-        c2 = Ops<R>::div(q.v[IP] * R(kp.gamma0), q.v[IR]);
-      const double inv = inv_dt_hyp_cs(q, Ops<R>::sqrt_(c2), kp, divx, divy);
-      if (inv > r.inv) r.inv = inv;  // NaN never wins: the reference's fmax-based Max ignores it
-    }
+    Ops_::finish_cell(gi, j, acc, r.u, r.u0, kp, io, divx, divy, r.neg_rho, r.neg_prs, r.nan_cnt, r.inv);
   }
 };
 

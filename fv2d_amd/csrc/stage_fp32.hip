@@ -43,11 +43,13 @@ struct BatchOcc {
 
 hipError_t launch_batch_fp32(const StageClass &c, const BatchJob *jobs, const BatchItem *items, const int *range,
                              int *counter, int stage, int grid, hipStream_t st) {
+  if (c.nw == 0) return launch_batch_march_fp32(c, jobs, items, range, counter, stage, grid, st);
   BatchLaunch f{jobs, items, range, counter, stage, grid, st, c.nw};
   return with_class(c, f);
 }
 
 int batch_occupancy_fp32(const StageClass &c) {
+  if (c.nw == 0) return batch_occupancy_march_fp32(c);
   BatchOcc f{c.nw};
   return with_class(c, f);
 }

@@ -268,9 +268,9 @@ def fifo_latencies(specs: list[JobSpec], service: dict) -> np.ndarray:
 
 # ------------------------------------------------------------------ autotuner
 
-# Tile candidates of the batched stage kernel: (segment height = rows per work item, chunk
-# rows = waves per workgroup).
-TILE_CANDIDATES = ((32, 4), (64, 4), (32, 8), (64, 8))
+# Tile candidates of the batched stage kernels: (segment height = rows per work item, chunk rows:
+# 0 the march kernel, 4 or 8 the strip kernel with that many waves per workgroup).
+TILE_CANDIDATES = ((16, 0), (8, 0), (24, 0), (32, 0), (64, 4))
 
 
 def _time_batch(specs_params, config: BatchConfig, launches: int = 3, warm: int = 1, lib=None) -> float:
@@ -290,7 +290,7 @@ def _time_batch(specs_params, config: BatchConfig, launches: int = 3, warm: int 
 
 
 def autotune(precision: int = FP32, sizes=SERVE_SIZES, kinds=KINDS, target_cells: int = 12 << 20,
-             tiles=TILE_CANDIDATES, blocks_per_cu=(0, 3, 2), mix_tiles=((64, 4), (64, 8)), cache: str | None = None,
+             tiles=TILE_CANDIDATES, blocks_per_cu=(0, 3, 2), mix_tiles=((16, 0), (24, 0), (64, 4)), cache: str | None = None,
              lib=None, log=None, use_graph: int = 1) -> dict:
     """Choose the tile of the batched stage kernel per kernel class (setup) and grid: the
     segment height (rows per work item) and the chunk height (rows per chunk = waves per
@@ -313,7 +313,7 @@ def autotune(precision: int = FP32, sizes=SERVE_SIZES, kinds=KINDS, target_cells
             copies = max(1, min(256, target_cells // (nx * ny)))
             best, best_rate = tiles[0], -1.0
             for seg, nw in tiles:
-                if seg > (ny + nw - 1) // nw * nw and (seg, nw) != tiles[0]:
+                if seg > ny + max(nw - 1, 0) and (seg, nw) != tiles[0]:
                     continue
                 p = job_params(spec, precision, seg, nw)
                 cfg = BatchConfig.defaults(precision=precision, max_jobs=max(copies, 1), use_graph=use_graph)
