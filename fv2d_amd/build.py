@@ -46,6 +46,7 @@ UNITS = [
     ("fv2d_capi.hip", ["-ffp-contract=off"]),
     ("fv2d_batch.hip", ["-ffp-contract=off"]),
     ("fv2d_noalloc.hip", ["-ffp-contract=off"]),
+    ("fv2d_xfer.hip", []),
 ]
 
 

@@ -34,6 +34,7 @@
 #include "fv2d_device.h"
 #include "fv2d_march_device.h"
 #include "fv2d_params.h"
+#include "fv2d_xfer.h"
 
 using namespace fv2d;
 
@@ -251,6 +252,7 @@ struct fv2d_batch {
   int total_items = 0;
   int64_t next_id = 1;
   bool dirty = true;
+  bool copies = false;  // holds a reference to the pinned copy buffers
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   int graph_classes = -1;
@@ -440,6 +442,7 @@ void fv2d_batch_destroy(fv2d_batch *b) {
   if (b->h_ctl) (void)hipHostFree(b->h_ctl);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   if (b->io) (void)hipStreamDestroy(b->io);
+  if (b->copies) copy_release(b->device);
   (void)hipSetDevice(cur);
   delete b;
 }
@@ -482,6 +485,8 @@ int fv2d_batch_create(const fv2d_batch_config *c, fv2d_batch **out) {
   };
   hipError_t e;
   if ((e = hipGetDevice(&b->device)) != hipSuccess) return fail("hipGetDevice", e);
+  copy_retain(b->device);
+  b->copies = true;
   if ((e = hipDeviceGetAttribute(&b->ncu, hipDeviceAttributeMultiprocessorCount, b->device)) != hipSuccess)
     return fail("CU count", e);
   if ((e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking)) != hipSuccess) return fail("stream", e);
@@ -600,7 +605,7 @@ int fv2d_batch_submit(fv2d_batch *b, const fv2d_params *p, const fv2d_problem *p
     BHIP(b, hipStreamSynchronize(b->stream));
   }
   if (q) {
-    BHIP(b, hipMemcpyAsync(b->d_upload, q, sizeof(double) * 4 * n, hipMemcpyHostToDevice, b->stream));
+    BHIP(b, copy_to_device(b->d_upload, q, sizeof(double) * 4 * n, b->device, b->stream));
     if (f32)
       hipLaunchKernelGGL(init_state_kernel<float>, dim3(grid_1d(n)), dim3(AUX_THREADS), 0, b->stream, J.kp,
                          b->d_upload, (float *)J.U, (float *)J.Q0);
@@ -796,7 +801,7 @@ int fv2d_batch_collect(fv2d_batch *b, int64_t id, double *q, double sums[4], fv2
       hipLaunchKernelGGL(get_prim_kernel<double>, dim3(grid_1d(n)), dim3(AUX_THREADS), 0, b->io, J.kp,
                          (const double *)src, fresh ? 1 : 0, b->d_out);
     BHIP(b, hipGetLastError());
-    BHIP(b, hipMemcpyAsync(q, b->d_out, sizeof(double) * 4 * n, hipMemcpyDeviceToHost, b->io));
+    BHIP(b, copy_to_host(q, b->d_out, sizeof(double) * 4 * n, b->device, b->io));
   }
   if (sums) {
     const void *u = in_us ? J.Us : J.U;

@@ -20,6 +20,7 @@
 #include "fv2d_device.h"
 #include "fv2d_params.h"
 #include "fv2d_sim.h"
+#include "fv2d_xfer.h"
 
 using namespace fv2d;
 
@@ -34,6 +35,7 @@ struct fv2d_handle {
   double *dts_log = nullptr;
   int dts_cap = 0;
   bool have_state = false;
+  bool copies = false;  // holds a reference to the pinned copy buffers
   unsigned long long last_counts[3] = {0, 0, 0};
   // stage-kernel timing (fv2d_profile): event pairs recorded since the last read
   bool prof = false;
@@ -155,6 +157,7 @@ void fv2d_destroy(fv2d_handle *h) {
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   if (h->d.stream) (void)hipStreamDestroy(h->d.stream);
+  if (h->copies) copy_release(h->device);
   (void)hipSetDevice(cur);
   delete h;
 }
@@ -187,6 +190,8 @@ int fv2d_create(const fv2d_params *p, fv2d_handle **out) {
   };
   hipError_t e;
   if ((e = hipGetDevice(&h->device)) != hipSuccess) return fail("hipGetDevice", e);
+  copy_retain(h->device);
+  h->copies = true;
   if ((e = hipStreamCreateWithFlags(&h->d.stream, hipStreamNonBlocking)) != hipSuccess) return fail("stream", e);
   const size_t state_bytes = 4 * (size_t)h->d.kp.plane * h->esize;
   if ((e = hipMalloc(&h->d.U, state_bytes)) != hipSuccess) return fail("hipMalloc U", e);
@@ -228,7 +233,7 @@ int fv2d_set_prim(fv2d_handle *h, const double *q) {
   int rc;
   if ((rc = ensure_staging(h))) return rc;
   const long long n = (long long)h->d.p.Nx * h->d.p.Ny;
-  HIPH(h, hipMemcpyAsync(h->staging, q, sizeof(double) * 4 * n, hipMemcpyHostToDevice, h->d.stream));
+  SIMH(h, copy_to_device(h->staging, q, sizeof(double) * 4 * n, h->device, h->d.stream));
   if (is_fp32(h))
     hipLaunchKernelGGL(init_state_kernel<float>, dim3(grid_1d(n)), dim3(AUX_THREADS), 0, h->d.stream, h->d.kp, h->staging,
                        (float *)h->d.U, (float *)h->d.Q0);
@@ -375,8 +380,7 @@ int fv2d_get_prim(fv2d_handle *h, double *q) {
     hipLaunchKernelGGL(get_prim_kernel<double>, dim3(grid_1d(n)), dim3(AUX_THREADS), 0, h->d.stream, h->d.kp,
                        (const double *)src, h->d.fresh_q0 ? 1 : 0, h->staging);
   HIPH(h, hipGetLastError());
-  HIPH(h, hipMemcpyAsync(q, h->staging, sizeof(double) * 4 * n, hipMemcpyDeviceToHost, h->d.stream));
-  HIPH(h, hipStreamSynchronize(h->d.stream));
+  SIMH(h, copy_to_host(q, h->staging, sizeof(double) * 4 * n, h->device, h->d.stream));
   return FV2D_OK;
 }
 
@@ -395,8 +399,7 @@ int fv2d_get_cons(fv2d_handle *h, double *u) {
     hipLaunchKernelGGL(get_cons_kernel<double>, dim3(grid_1d(n)), dim3(AUX_THREADS), 0, h->d.stream, h->d.kp,
                        (const double *)h->d.U, h->staging);
   HIPH(h, hipGetLastError());
-  HIPH(h, hipMemcpyAsync(u, h->staging, sizeof(double) * 4 * n, hipMemcpyDeviceToHost, h->d.stream));
-  HIPH(h, hipStreamSynchronize(h->d.stream));
+  SIMH(h, copy_to_host(u, h->staging, sizeof(double) * 4 * n, h->device, h->d.stream));
   return FV2D_OK;
 }
 
