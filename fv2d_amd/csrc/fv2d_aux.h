@@ -68,28 +68,6 @@ __global__ void __launch_bounds__(256) dt_cells_kernel(KParams kp, const S *src,
     partials[blockIdx.x] = b;
 }
 
-// Loop control of main.cpp:62-83 for one step, given the reduced hyperbolic inverse dt:
-// while t + epsilon < tend: dt = CFL / max(inv_hyp, inv_tc, inv_visc) (ComputeDt.h:64), take
-// the step, t += dt. Sets ctl->active = 0 when the loop has ended.
-__device__ inline void advance_control(StepCtl *ctl, double inv_hyp, const KParams &kp, double *dts_log) {
-  const bool go = (ctl->t + kp.epsilon < ctl->tend) && (ctl->max_steps <= 0 || ctl->nsteps < ctl->max_steps);
-  if (!go) {
-    ctl->active = 0;
-    return;
-  }
-  double mm = inv_hyp;  // std::max({hyp, tc, visc}) keeps the first of equal maxima
-  if (mm < kp.inv_tc) mm = kp.inv_tc;
-  if (mm < kp.inv_visc) mm = kp.inv_visc;
-  const double dt = kp.CFL / mm;
-  ctl->dt = dt;
-  ctl->dt_dx = dt / kp.dx;
-  ctl->dt_dy = dt / kp.dy;
-  ctl->t = ctl->t + dt;
-  if (dts_log) dts_log[ctl->nsteps] = dt;
-  ctl->nsteps = ctl->nsteps + 1;
-  ctl->active = 1;
-}
-
 // Reduce the partial maxima into ctl->inv_hyp; in advance mode also run the loop control.
 static __global__ __attribute__((unused)) void __launch_bounds__(1024) reduce_kernel(StepCtl *ctl, const double *partials, int nparts,
                                                              KParams kp, int advance, double *dts_log) {
@@ -106,23 +84,22 @@ static __global__ __attribute__((unused)) void __launch_bounds__(1024) reduce_ke
   if (advance) advance_control(ctl, b, kp, dts_log);
 }
 
-// The same for the march kernel (one wave): its slots keep the maximum of the current state
-// until a step that replaces the state begins.
-static __global__ __attribute__((unused)) void __launch_bounds__(64) reduce_acc_kernel(StepCtl *ctl, unsigned long long *acc, KParams kp,
-                                                              int advance, double *dts_log) {
+// For the march kernel (one wave): the control block *cur and the maximum over the slots of its state
+// into ctl (which holds the reset counters) and, when given, into the host's copy.
+static __global__ __attribute__((unused)) void __launch_bounds__(64) report_kernel(StepCtl *ctl, const StepCtl *cur, const unsigned long long *acc,
+                                                          StepCtl *host) {
   const double b = acc_read(acc);
-  const bool was = ctl->active != 0;
-  if (threadIdx.x == 0) {
-    ctl->inv_hyp = b;
-    if (advance && was) advance_control(ctl, b, kp, dts_log);
-  }
-  __syncthreads();
-  if (advance && was && ctl->active) acc_clear(acc);
+  if (threadIdx.x != 0) return;
+  StepCtl c = *cur;
+  c.inv_hyp = b;
+  c.neg_rho = ctl->neg_rho;
+  c.neg_prs = ctl->neg_prs;
+  c.nan_cnt = ctl->nan_cnt;
+  *ctl = c;
+  if (host) *host = c;
 }
 
-static __global__ __attribute__((unused)) void __launch_bounds__(64) set_dt_kernel(StepCtl *ctl, unsigned long long *acc, double dt, double dx, double dy) {
-  if (acc) acc_clear(acc);
-  if (threadIdx.x != 0) return;
+static __global__ __attribute__((unused)) void set_dt_kernel(StepCtl *ctl, double dt, double dx, double dy) {
   ctl->dt = dt;
   ctl->dt_dx = dt / dx;
   ctl->dt_dy = dt / dy;
@@ -138,7 +115,8 @@ static __global__ __attribute__((unused)) void set_loop_kernel(StepCtl *ctl, dou
 }
 
 static __global__ __attribute__((unused)) void __launch_bounds__(64) clear_ctl_kernel(StepCtl *ctl, unsigned long long *acc) {
-  if (acc) acc_clear(acc);
+  if (acc)
+    for (int k = 0; k < 3; ++k) acc_clear(acc + k * ACC_WORDS);
   if (threadIdx.x != 0) return;
   ctl->dt = ctl->dt_dx = ctl->dt_dy = 0.0;
   ctl->t = ctl->tend = 0.0;

@@ -34,6 +34,9 @@ struct fv2d_handle {
   double *sums = nullptr;     // 4 doubles
   double *dts_log = nullptr;
   int dts_cap = 0;
+  // the control block as of the last call that changed the state: every such call ends by bringing it
+  // to the host, so the dt of the current state is known there
+  StepCtl now = {};
   bool have_state = false;
   bool copies = false;  // holds a reference to the pinned copy buffers
   unsigned long long last_counts[3] = {0, 0, 0};
@@ -157,6 +160,7 @@ void fv2d_destroy(fv2d_handle *h) {
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   if (h->d.stream) (void)hipStreamDestroy(h->d.stream);
+  if (h->d.host_ctl) (void)hipHostFree(h->d.host_ctl);
   if (h->copies) copy_release(h->device);
   (void)hipSetDevice(cur);
   delete h;
@@ -197,12 +201,15 @@ int fv2d_create(const fv2d_params *p, fv2d_handle **out) {
   if ((e = hipMalloc(&h->d.U, state_bytes)) != hipSuccess) return fail("hipMalloc U", e);
   if ((e = hipMalloc(&h->d.Us, state_bytes)) != hipSuccess) return fail("hipMalloc Us", e);
   if ((e = hipMalloc(&h->d.Q0, state_bytes)) != hipSuccess) return fail("hipMalloc Q0", e);
-  if ((e = hipMalloc((void **)&h->d.ctl, sizeof(StepCtl))) != hipSuccess) return fail("hipMalloc ctl", e);
+  if ((e = hipMalloc((void **)&h->d.ctl, 2 * sizeof(StepCtl))) != hipSuccess) return fail("hipMalloc ctl", e);
   if ((e = hipMalloc((void **)&h->d.partials, sim_partials_bytes(h->d))) != hipSuccess)
     return fail("hipMalloc partials", e);
   if ((e = hipMalloc((void **)&h->rowsum, sizeof(double) * 4 * (size_t)p->Ny)) != hipSuccess)
     return fail("hipMalloc rowsum", e);
   if ((e = hipMalloc((void **)&h->sums, sizeof(double) * 4)) != hipSuccess) return fail("hipMalloc sums", e);
+  if (h->d.march.ntasks &&
+      (e = hipHostMalloc((void **)&h->d.host_ctl, sizeof(StepCtl), hipHostMallocDefault)) != hipSuccess)
+    return fail("pinned control block", e);
   if (p->gravity_mode == FV2D_GRAV_ANALYTICAL) {
     // getAnalyticalGravity (Gravity.h:15-30) depends on the row only; evaluated here with
     // the host libm and passed through float, as getGravity returns float.
@@ -241,10 +248,10 @@ int fv2d_set_prim(fv2d_handle *h, const double *q) {
     hipLaunchKernelGGL(init_state_kernel<double>, dim3(grid_1d(n)), dim3(AUX_THREADS), 0, h->d.stream, h->d.kp,
                        h->staging, (double *)h->d.U, (double *)h->d.Q0);
   HIPH(h, hipGetLastError());
+  h->d.cur = h->d.set = 0;
   hipLaunchKernelGGL(clear_ctl_kernel, dim3(1), dim3(64), 0, h->d.stream, h->d.ctl, sim_acc(h->d));
   SIMH(h, sim_launch_dt_tiles(h->d, h->d.Q0, 1));
-  SIMH(h, sim_launch_reduce(h->d, 0, nullptr));
-  HIPH(h, hipStreamSynchronize(h->d.stream));
+  SIMH(h, sim_finish(h->d, h->now));
   h->have_state = true;
   h->d.fresh_q0 = true;
   memset(h->last_counts, 0, sizeof h->last_counts);
@@ -265,10 +272,10 @@ int fv2d_set_problem(fv2d_handle *h, const fv2d_problem *prob) {
     hipLaunchKernelGGL(problem_ic_kernel<double>, dim3(grid_1d(n)), dim3(AUX_THREADS), 0, h->d.stream, h->d.kp, a,
                        (double *)h->d.U, (double *)h->d.Q0);
   HIPH(h, hipGetLastError());
+  h->d.cur = h->d.set = 0;
   hipLaunchKernelGGL(clear_ctl_kernel, dim3(1), dim3(64), 0, h->d.stream, h->d.ctl, sim_acc(h->d));
   SIMH(h, sim_launch_dt_tiles(h->d, h->d.Q0, 1));
-  SIMH(h, sim_launch_reduce(h->d, 0, nullptr));
-  HIPH(h, hipStreamSynchronize(h->d.stream));
+  SIMH(h, sim_finish(h->d, h->now));
   h->have_state = true;
   h->d.fresh_q0 = true;
   memset(h->last_counts, 0, sizeof h->last_counts);
@@ -279,10 +286,7 @@ int fv2d_compute_dt(fv2d_handle *h, double *dt, double inv[3]) {
   if (!h) return FV2D_E_INVALID;
   if (!h->have_state) FAILH(h, FV2D_E_STATE, "fv2d_compute_dt: no state (call fv2d_set_prim first)");
   HIPH(h, hipSetDevice(h->device));
-  StepCtl c;
-  HIPH(h, hipMemcpyAsync(&c, h->d.ctl, sizeof c, hipMemcpyDeviceToHost, h->d.stream));
-  HIPH(h, hipStreamSynchronize(h->d.stream));
-  const double a = c.inv_hyp, b = h->d.kp.inv_tc, d = h->d.kp.inv_visc;
+  const double a = h->now.inv_hyp, b = h->d.kp.inv_tc, d = h->d.kp.inv_visc;
   double m = a;
   if (m < b) m = b;
   if (m < d) m = d;
@@ -295,29 +299,19 @@ int fv2d_compute_dt(fv2d_handle *h, double *dt, double inv[3]) {
   return FV2D_OK;
 }
 
-static int read_counts(fv2d_handle *h, unsigned long long tot[3]) {
-  StepCtl c;
-  HIPH(h, hipMemcpyAsync(&c, h->d.ctl, sizeof c, hipMemcpyDeviceToHost, h->d.stream));
-  HIPH(h, hipStreamSynchronize(h->d.stream));
-  tot[0] = c.neg_rho;
-  tot[1] = c.neg_prs;
-  tot[2] = c.nan_cnt;
-  return FV2D_OK;
-}
-
 int fv2d_step(fv2d_handle *h, double dt, fv2d_step_stats *stats) {
   if (!h) return FV2D_E_INVALID;
   if (!h->have_state) FAILH(h, FV2D_E_STATE, "fv2d_step: no state (call fv2d_set_prim first)");
   HIPH(h, hipSetDevice(h->device));
-  hipLaunchKernelGGL(set_dt_kernel, dim3(1), dim3(64), 0, h->d.stream, h->d.ctl, sim_acc(h->d), dt, h->d.kp.dx, h->d.kp.dy);
-  HIPH(h, hipGetLastError());
+  if (!h->d.march.ntasks) {
+    hipLaunchKernelGGL(set_dt_kernel, dim3(1), dim3(1), 0, h->d.stream, h->d.ctl, dt, h->d.kp.dx, h->d.kp.dy);
+    HIPH(h, hipGetLastError());
+  }
   bool swapped;
-  int rc;
-  SIMH(h, sim_enqueue_step(h->d, h->d.fresh_q0, swapped));
-  SIMH(h, sim_launch_reduce(h->d, 0, nullptr));
+  SIMH(h, sim_enqueue_step(h->d, h->d.fresh_q0, swapped, MARCH_GIVEN, dt, nullptr));
   h->d.fresh_q0 = false;
-  unsigned long long tot[3];
-  if ((rc = read_counts(h, tot))) return rc;
+  SIMH(h, sim_finish(h->d, h->now));
+  const unsigned long long tot[3] = {h->now.neg_rho, h->now.neg_prs, h->now.nan_cnt};
   if (stats) {
     stats->negative_density = tot[0] - h->last_counts[0];
     stats->negative_pressure = tot[1] - h->last_counts[1];
@@ -346,7 +340,8 @@ int fv2d_advance(fv2d_handle *h, double *t, double tend, int32_t max_steps, doub
     h->dts_cap = max_steps;
   }
   StepCtl c;
-  SIMH(h, sim_advance(h->d, *t, tend, max_steps, dts ? h->dts_log : nullptr, c));
+  SIMH(h, sim_advance(h->d, *t, tend, max_steps, h->now.inv_hyp, dts ? h->dts_log : nullptr, c));
+  h->now = c;
   const int done = c.nsteps;
   if (dts && done > 0) {
     HIPH(h, hipMemcpyAsync(dts, h->dts_log, sizeof(double) * done, hipMemcpyDeviceToHost, h->d.stream));

@@ -39,6 +39,28 @@ __device__ inline double acc_read(const unsigned long long *acc) {
 }
 __device__ inline void acc_clear(unsigned long long *acc) { acc[(threadIdx.x & 63) * ACC_STRIDE] = 0ull; }
 
+// Loop control of main.cpp:62-83 for one step, given the reduced hyperbolic inverse dt:
+// while t + epsilon < tend: dt = CFL / max(inv_hyp, inv_tc, inv_visc) (ComputeDt.h:64), take
+// the step, t += dt. Sets ctl->active = 0 when the loop has ended.
+__device__ inline void advance_control(StepCtl *ctl, double inv_hyp, const KParams &kp, double *dts_log) {
+  const bool go = (ctl->t + kp.epsilon < ctl->tend) && (ctl->max_steps <= 0 || ctl->nsteps < ctl->max_steps);
+  if (!go) {
+    ctl->active = 0;
+    return;
+  }
+  double mm = inv_hyp;  // std::max({hyp, tc, visc}) keeps the first of equal maxima
+  if (mm < kp.inv_tc) mm = kp.inv_tc;
+  if (mm < kp.inv_visc) mm = kp.inv_visc;
+  const double dt = kp.CFL / mm;
+  ctl->dt = dt;
+  ctl->dt_dx = dt / kp.dx;
+  ctl->dt_dy = dt / kp.dy;
+  ctl->t = ctl->t + dt;
+  if (dts_log) dts_log[ctl->nsteps] = dt;
+  ctl->nsteps = ctl->nsteps + 1;
+  ctl->active = 1;
+}
+
 // Epilogue commit: reset counters (rare, atomics) and the workgroup's max inverse dt into
 // partials[blk] (no atomics on the hot value: the reduction kernel reads all partials).
 template <int NT>

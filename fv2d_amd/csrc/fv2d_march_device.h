@@ -123,11 +123,70 @@ __device__ inline void march_task(const KParams &kp, const StageIO<S> &io, const
 }
 
 
+// How a stage of a single simulation gets its dt. The first stage of a step runs the loop control
+// itself: each of its waves takes the maximum over the slots of the previous state and forms the
+// same dt, and the wave of task 0 records it for the second stage and the next step, which read it
+// after the launch boundary. A launch of its own for this took 4.2 us of every step. Control blocks
+// alternate, the slots go round three sets: read by the step, filled by it, cleared for the next.
+enum : int { MARCH_READ = 0, MARCH_ADVANCE = 1, MARCH_GIVEN = 2 };
+struct MarchCtl {
+  int mode;           // MARCH_READ: the step's dt is in `out`; else begin the step
+  const StepCtl *in;  // control block of the previous step (MARCH_ADVANCE)
+  StepCtl *out;       // of this step
+  const unsigned long long *acc_in;  // slots of the state the step starts from (MARCH_ADVANCE)
+  unsigned long long *acc_clear;     // slots the next step will fill
+  double *dts_log;
+  double dt;  // MARCH_GIVEN
+};
+
+// The step's dt, dt/dx, dt/dy; false when the loop has ended. acc: the slots this step fills.
+__device__ inline bool march_begin(const MarchCtl &m, const KParams &kp, unsigned long long *acc, int task, double &dt,
+                                   double &dt_dx, double &dt_dy) {
+  if (m.mode == MARCH_READ) {
+    dt = uni(m.out->dt);
+    dt_dx = uni(m.out->dt_dx);
+    dt_dy = uni(m.out->dt_dy);
+    return uni(m.out->active) != 0;
+  }
+  StepCtl c;
+  if (m.mode == MARCH_ADVANCE) {
+    c = *m.in;
+    if (c.active) advance_control(&c, acc_read(m.acc_in), kp, task == 0 && (threadIdx.x & 63) == 0 ? m.dts_log : nullptr);
+  } else {
+    c.dt = m.dt;
+    c.dt_dx = m.dt / kp.dx;
+    c.dt_dy = m.dt / kp.dy;
+    c.t = c.tend = 0.0;
+    c.active = 1;
+    c.nsteps = c.max_steps = 0;
+  }
+  if (task == 0) {
+    if ((threadIdx.x & 63) == 0) {
+      StepCtl *o = m.out;  // (the reset counters and the reduced maximum are not part of the step)
+      o->dt = c.dt;
+      o->dt_dx = c.dt_dx;
+      o->dt_dy = c.dt_dy;
+      o->t = c.t;
+      o->tend = c.tend;
+      o->active = c.active;
+      o->nsteps = c.nsteps;
+      o->max_steps = c.max_steps;
+    }
+    acc_clear(m.acc_clear);
+    if (!c.active) {  // no step: the state and its maximum stay
+      const int s = (threadIdx.x & 63) * ACC_STRIDE;
+      acc[s] = m.acc_in[s];
+    }
+  }
+  dt = uni(c.dt);
+  dt_dx = uni(c.dt_dx);
+  dt_dy = uni(c.dt_dy);
+  return uni(c.active) != 0;
+}
+
 template <class K, typename R, typename S>
 __global__ void __launch_bounds__(64 * MARCH_WAVES) __attribute__((amdgpu_waves_per_eu(K::kWPE, K::kWPE)))
-march_kernel(const KParams kp, const StageIO<S> io, const MarchGeom g) {
-  const StepCtl *ctl = io.ctl;
-  if (!uni(ctl->active)) return;  // the device loop has ended
+march_kernel(const KParams kp, const StageIO<S> io, const MarchGeom g, const MarchCtl mc) {
   // XCD x (blocks b with b % 8 == x) takes a contiguous run of blocks, so that neighbouring
   // strips, which share halo columns, run on one L2
   const int nb = gridDim.x, q = nb >> 3, rem = nb & 7;
@@ -135,7 +194,9 @@ march_kernel(const KParams kp, const StageIO<S> io, const MarchGeom g) {
   const int blk = x * q + (x < rem ? x : rem) + k;
   const int task = blk * MARCH_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (task >= g.ntasks) return;
-  march_task<K, R, S>(kp, io, g, task, uni(ctl->dt), uni(ctl->dt_dx), uni(ctl->dt_dy));
+  double dt, dt_dx, dt_dy;
+  if (!march_begin(mc, kp, io.acc, task, dt, dt_dx, dt_dy)) return;  // the device loop has ended
+  march_task<K, R, S>(kp, io, g, task, dt, dt_dx, dt_dy);
 }
 
 // Batched stage: the waves of a persistent grid run the (job, task) pairs of one kernel class, each
@@ -182,20 +243,21 @@ struct MarchLaunch {
   const KParams &kp;
   const StageIO<S> &io;
   const MarchGeom &g;
+  const MarchCtl &mc;
   hipStream_t st;
   template <int RC, int RM, bool TC, bool VI, bool XG>
   hipError_t operator()() {
     typedef MarchStage<R, S, RC, RM, TC, VI, XG, DIVF> K;
     hipLaunchKernelGGL((march_kernel<K, R, S>), dim3((g.ntasks + MARCH_WAVES - 1) / MARCH_WAVES),
-                       dim3(64 * MARCH_WAVES), 0, st, kp, io, g);
+                       dim3(64 * MARCH_WAVES), 0, st, kp, io, g, mc);
     return hipGetLastError();
   }
 };
 
 template <typename R, typename S, int DIVF>
 hipError_t launch_march(const StageClass &c, const KParams &kp, const StageIO<S> &io, const MarchGeom &g,
-                        hipStream_t st) {
-  MarchLaunch<R, S, DIVF> f{kp, io, g, st};
+                        const MarchCtl &mc, hipStream_t st) {
+  MarchLaunch<R, S, DIVF> f{kp, io, g, mc, st};
   return with_class(c, f);
 }
 
@@ -229,11 +291,11 @@ struct BatchMarchOcc {
 };
 
 // Defined in march_fp64.hip / march_fp64_exact.hip / march_fp32.hip.
-hipError_t launch_march_fp64(const StageClass &c, const KParams &kp, const StageIO<double> &io, const MarchGeom &g,
-                             hipStream_t st);
+hipError_t launch_march_fp64(const StageClass &c, const KParams &kp, const StageIO<double> &io,
+                             const MarchGeom &g, const MarchCtl &mc, hipStream_t st);
 hipError_t launch_march_fp64_exact(const StageClass &c, const KParams &kp, const StageIO<double> &io,
-                                   const MarchGeom &g, hipStream_t st);
-hipError_t launch_march_fp32(const StageClass &c, const KParams &kp, const StageIO<float> &io, const MarchGeom &g,
-                             hipStream_t st);
+                             const MarchGeom &g, const MarchCtl &mc, hipStream_t st);
+hipError_t launch_march_fp32(const StageClass &c, const KParams &kp, const StageIO<float> &io,
+                             const MarchGeom &g, const MarchCtl &mc, hipStream_t st);
 
 }  // namespace fv2d

@@ -40,8 +40,8 @@ constexpr size_t NA_STATE = NA_GRAV + sizeof(float) * FV2D_NOALLOC_MAX_ROWS;    
 constexpr size_t NA_STATE_BYTES = 4 * sizeof(double) * (size_t)FV2D_NOALLOC_MAX_PLANE;  // one state, FP64
 constexpr size_t NA_BYTES = NA_STATE + 3 * NA_STATE_BYTES;
 static_assert(NA_DTS % 256 == 0 && NA_GRAV % 256 == 0 && NA_STATE % 256 == 0, "scratch regions must stay aligned");
-static_assert(sizeof(StepCtl) <= NA_PARTS, "control block region too small");
-static_assert(ACC_WORDS <= FV2D_NOALLOC_MAX_WORKGROUPS, "the dt slots share the partials' region");
+static_assert(2 * sizeof(StepCtl) <= NA_PARTS, "control block region too small");
+static_assert(3 * ACC_WORDS <= FV2D_NOALLOC_MAX_WORKGROUPS, "the dt slots share the partials' region");
 
 }  // namespace
 
@@ -161,12 +161,12 @@ int fv2d_run_noalloc(const fv2d_params *p, const double *q_in, double *q_out, do
   hipLaunchKernelGGL(clear_ctl_kernel, dim3(1), dim3(64), 0, d.stream, d.ctl, sim_acc(d));
   NA_HIP(hipGetLastError());
   NA_HIP(sim_launch_dt_tiles(d, d.Q0, 1));
-  NA_HIP(sim_launch_reduce(d, 0, nullptr));
+  if (!d.march.ntasks) NA_HIP(sim_launch_reduce(d, 0, nullptr));
   d.fresh_q0 = true;
 
   // fv2d_advance
   StepCtl c;
-  NA_HIP(sim_advance(d, *t, tend, max_steps, dts_log, c));
+  NA_HIP(sim_advance(d, *t, tend, max_steps, 0.0, dts_log, c));
   if (dts && c.nsteps > 0)
     NA_HIP(hipMemcpyAsync(dts, dts_log, sizeof(double) * c.nsteps, hipMemcpyDeviceToHost, d.stream));
 

@@ -4,8 +4,8 @@
 namespace fv2d {
 
 hipError_t launch_march_fp32(const StageClass &c, const KParams &kp, const StageIO<float> &io, const MarchGeom &g,
-                             hipStream_t st) {
-  return launch_march<float, float, DIVF_RUNTIME>(c, kp, io, g, st);
+                             const MarchCtl &mc, hipStream_t st) {
+  return launch_march<float, float, DIVF_RUNTIME>(c, kp, io, g, mc, st);
 }
 
 }  // namespace fv2d

@@ -6,9 +6,9 @@
 namespace fv2d {
 
 hipError_t launch_march_fp64(const StageClass &c, const KParams &kp, const StageIO<double> &io, const MarchGeom &g,
-                             hipStream_t st) {
-  if (kp.divx == DIV_EXACT && kp.divy == DIV_EXACT) return launch_march_fp64_exact(c, kp, io, g, st);
-  return launch_march<double, double, DIVF_GENERAL>(c, kp, io, g, st);
+                             const MarchCtl &mc, hipStream_t st) {
+  if (kp.divx == DIV_EXACT && kp.divy == DIV_EXACT) return launch_march_fp64_exact(c, kp, io, g, mc, st);
+  return launch_march<double, double, DIVF_GENERAL>(c, kp, io, g, mc, st);
 }
 
 }  // namespace fv2d

@@ -5,8 +5,9 @@
 namespace fv2d {
 
 hipError_t launch_march_fp64_exact(const StageClass &c, const KParams &kp, const StageIO<double> &io,
-                                   const MarchGeom &g, hipStream_t st) {
-  return launch_march<double, double, DIVF_EXACT>(c, kp, io, g, st);
+                                   const MarchGeom &g,
+                             const MarchCtl &mc, hipStream_t st) {
+  return launch_march<double, double, DIVF_EXACT>(c, kp, io, g, mc, st);
 }
 
 }  // namespace fv2d
