@@ -267,8 +267,8 @@ FV2D_HD St<R> cons_to_prim(const St<R> &u, R gm1, const DivBy<R> &byr) {
   byr.template all<2>(m, w);
   r.v[IU] = w[0];
   r.v[IV] = w[1];
-  R Ek = R(0.5) * r.v[IR] * (r.v[IU] * r.v[IU] + r.v[IV] * r.v[IV]);
-  r.v[IP] = (u.v[IE] - Ek) * gm1;
+  // one expression, so that the FP32 form subtracts the kinetic energy unrounded (one FMA)
+  r.v[IP] = (u.v[IE] - R(0.5) * r.v[IR] * (r.v[IU] * r.v[IU] + r.v[IV] * r.v[IV])) * gm1;
   return r;
 }
 template <typename R>
