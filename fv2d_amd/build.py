@@ -41,6 +41,7 @@ UNITS = [
     ("march_fp64.hip", ["-ffp-contract=off"]),
     ("march_fp64_exact.hip", ["-ffp-contract=off"]),
     ("march_fp32.hip", ["-ffp-contract=on"]),
+    ("march_fp32s64.hip", ["-ffp-contract=on"]),
     ("march_batch_fp64.hip", ["-ffp-contract=off"]),
     ("march_batch_fp32.hip", ["-ffp-contract=on"]),
     ("fv2d_capi.hip", ["-ffp-contract=off"]),

@@ -641,7 +641,7 @@ int fv2d_batch_submit(fv2d_batch *b, const fv2d_params *p, const fv2d_problem *p
     dj.nblocks = mg.ntasks;
     dj.seg = mg.seg;
     dj.nsx = mg.nsx;
-    dj.nsy = mg.nsy;
+    dj.nsy = mg.ntasks / mg.nsx;
     dj.march = 1;
   }
   dj.U = J.U;

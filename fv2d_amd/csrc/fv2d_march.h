@@ -25,32 +25,55 @@ namespace fv2d {
 
 constexpr int MARCH_OUT = 60;  // output columns per wave
 
-// Waves per SIMD of the kernels: FP64 84-128 VGPRs (4 waves), FP32 at most 80 (6 waves), or 96
-// (5 waves) where the gravity and wall terms come with viscosity or conduction (they spill at 80).
-FV2D_HD constexpr int march_wpe(bool fp64, bool xg_parabolic) { return fp64 ? 4 : (xg_parabolic ? 5 : 6); }
+// Waves per SIMD of the kernels: 4 with an FP64 state (84-128 VGPRs in FP64; FP32 on the FP64 state: 9.5
+// KB of LDS per wave), FP32 at most 80 VGPRs (6 waves), or 96 (5 waves) where the gravity and wall
+// terms come with viscosity or conduction (they spill at 80).
+FV2D_HD constexpr int march_wpe(bool state64, bool xg_parabolic) { return state64 ? 4 : (xg_parabolic ? 5 : 6); }
 
-// Work split of one grid: tasks (strip, segment of `seg` rows), one wave each.
+// Work split of one grid: tasks (strip, segment of rows), one wave each. The rows are one band, or 8
+// bands of `height` rows, one per XCD. A band's segments are `nlong` ones of `seg` rows from its first
+// row on, then short ones of `sseg` rows up to its end; task t of a band is strip t % nsx of segment
+// t / nsx. Tasks past a band's rows are empty. With one band all segments are long.
 struct MarchGeom {
-  int nsx, nsy;  // strips, segments
-  int seg;       // rows per segment
-  int ntasks;    // nsx * nsy
+  int nsx;
+  int bands, height;
+  int nlong, seg, sseg;
+  int per_band;  // tasks per band
+  int ntasks;    // bands * per_band
 };
 
 FV2D_HD MarchGeom march_geom(int Nx, int Ny, int seg) {
   MarchGeom g;
   g.nsx = (Nx + MARCH_OUT - 1) / MARCH_OUT;
-  g.seg = seg;
-  g.nsy = (Ny + seg - 1) / seg;
-  g.ntasks = g.nsx * g.nsy;
+  g.bands = 1;
+  g.height = Ny;
+  g.nlong = (Ny + seg - 1) / seg;
+  g.seg = g.sseg = seg;
+  g.per_band = g.ntasks = g.nsx * g.nlong;
   return g;
 }
 
-// Output columns from i0 and rows [jb, je) of a task.
-FV2D_HD void march_task_rows(const MarchGeom &g, int Ny, int task, int &i0, int &jb, int &je) {
-  const int sy = task / g.nsx;
-  i0 = (task - sy * g.nsx) * MARCH_OUT;
-  jb = sy * g.seg;
-  je = (jb + g.seg < Ny) ? jb + g.seg : Ny;
+FV2D_HD MarchGeom march_geom_banded(int Nx, int Ny, int nlong, int seg, int sseg) {
+  MarchGeom g = march_geom(Nx, Ny, seg);
+  g.bands = 8;
+  g.height = (Ny + 7) / 8;
+  g.nlong = nlong;
+  g.sseg = sseg;
+  const int rest = g.height - nlong * seg;
+  g.per_band = g.nsx * (nlong + (rest > 0 ? (rest + sseg - 1) / sseg : 0));
+  g.ntasks = 8 * g.per_band;
+  return g;
+}
+
+// Output columns from i0 and rows [jb, je) of task t of a band (je <= jb: an empty task).
+FV2D_HD void march_task_rows(const MarchGeom &g, int Ny, int band, int t, int &i0, int &jb, int &je) {
+  const int m = t / g.nsx;
+  i0 = (t - m * g.nsx) * MARCH_OUT;
+  const int b0 = band * g.height, b1 = (b0 + g.height < Ny) ? b0 + g.height : Ny;
+  const bool lng = m < g.nlong;
+  jb = b0 + (lng ? m * g.seg : g.nlong * g.seg + (m - g.nlong) * g.sseg);
+  je = jb + (lng ? g.seg : g.sseg);
+  je = je < b1 ? je : b1;
 }
 
 // A lane's own slots in LDS (device) or host memory; slot k of the lane is at [64 * k].
@@ -71,6 +94,7 @@ struct MarchLane {
   R um, vm;          // velocities of row j-1
   LanePtr<R> low;    // the lane's slots (stride 64) of the y face (j-1, j): flux, viscous terms,
                      // conduction flux, interface pressure
+  LanePtr<S> ring;   // the lane's slots of U of rows j .. j+2 (kRing)
   S raw[4];          // storage values of row j+2
   // within a row
   R q2[4], t2;       // primitives of row j+2
@@ -102,16 +126,17 @@ struct MarchStage : StageOps<R, S, TC, DIVF_> {
   typedef MarchLane<R, S> Lane;
   static constexpr bool kTC = TC, kVISC = VISC, kPLM = RECON == PLM;
   static constexpr bool kParkQ2 = sizeof(R) == 8;
-  // U of a row is kept from its load to its update, two rows later (FP32: the slots fit; reading it
-  // again took 30% of the HBM reads at 4096^2, where the rows in flight outgrow an XCD's 4 MB L2).
-  static constexpr bool kRing = sizeof(R) == 4 && sizeof(S) == 4;
-  static constexpr int kWPE = march_wpe(sizeof(R) == 8, XG && (TC || VISC));
+  // U of a row is kept from its load to its update, two rows later (the FP32 forms, where the slots
+  // fit): the rows in flight outgrow an XCD's 4 MB L2, so reading it again was a third of the HBM reads
+  // at 4096^2 (FP32 733 -> 491 MB per stage).
+  static constexpr bool kRing = sizeof(R) == 4;
+  static constexpr int NRING = kRing ? 12 : 0;
+  static constexpr int kWPE = march_wpe(sizeof(S) == 8, XG && (TC || VISC));
 
   // Slots of Lane::low.
   static constexpr int LFY = 0, LVY = 4, LFC = LVY + (VISC ? 3 : 0), LPY = LFC + (TC ? 1 : 0);
   static constexpr int LAL = LPY + (XG ? 1 : 0), LQ2 = LAL + 4;
-  static constexpr int LU = LQ2 + (kParkQ2 ? 5 : 0);  // U of rows j .. j+2, a ring of three
-  static constexpr int NLOW = LU + (kRing ? 12 : 0);
+  static constexpr int NLOW = LQ2 + (kParkQ2 ? 5 : 0);
 
   // The lane's column i0-2+lane, ghosts mapped to their source.
   static FV2D_HD void set_column(int lane, int i0, const KParams &kp, Lane &r) {
@@ -148,16 +173,16 @@ struct MarchStage : StageOps<R, S, TC, DIVF_> {
   }
   static FV2D_HD void ring_put(int j, const S raw[4], Lane &r) {
     if (!kRing) return;
-    const LanePtr<R> p = r.low + 64 * (LU + 4 * int((unsigned)j % 3u));
+    const LanePtr<S> p = r.ring + 64 * 4 * int((unsigned)j % 3u);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) p[64 * v] = R(raw[v]);
+    for (int v = 0; v < 4; ++v) p[64 * v] = raw[v];
   }
   // Own-cell U of row j (the other lanes read a column inside the grid and drop it).
   static FV2D_HD void load_own(int j, const KParams &kp, const StageIO<S> &io, const Lane &r, S u[4]) {
     if (kRing && io.qsrc != QSRC_Q0) {
-      const LanePtr<R> p = r.low + 64 * (LU + 4 * int((unsigned)j % 3u));
+      const LanePtr<S> p = r.ring + 64 * 4 * int((unsigned)j % 3u);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) u[v] = S(p[64 * v]);
+      for (int v = 0; v < 4; ++v) u[v] = p[64 * v];
       return;
     }
     const long long k = (long long)j * kp.pitch;

@@ -67,6 +67,7 @@ __device__ inline void march_rows(const KParams &kp, const StageIO<S> &io, int i
   }
   for (int j = jb; j < je; ++j) {
     r.low = opaque<R>(r.low);
+    if (K::kRing) r.ring = opaque<S>(r.ring);
     K::row_begin(j, kp, io, r);
 #pragma unroll
     for (int v = 0; v < 4; ++v) r.q0r[v] = shl1(r.q0[v]);
@@ -106,22 +107,23 @@ __device__ inline void march_rows(const KParams &kp, const StageIO<S> &io, int i
   }
 }
 
-// One wave's task of a stage.
+// One wave's task of a stage: rows [jb, je) of the strip at i0; `slot` picks its dt slot.
 template <class K, typename R, typename S>
-__device__ inline void march_task(const KParams &kp, const StageIO<S> &io, const MarchGeom &g, int task, double dt,
+__device__ inline void march_task(const KParams &kp, const StageIO<S> &io, int i0, int jb, int je, int slot, double dt,
                                   double dt_dx, double dt_dy) {
-  int i0, jb, je;
-  march_task_rows(g, kp.Ny, task, i0, jb, je);
   __shared__ R low[MARCH_WAVES][K::NLOW * 64];
   typename K::Lane r;
   r.low = (LanePtr<R>)(low[threadIdx.x >> 6] + (threadIdx.x & 63));
+  if constexpr (K::kRing) {
+    __shared__ S ring[MARCH_WAVES][K::NRING * 64];
+    r.ring = (LanePtr<S>)(ring[threadIdx.x >> 6] + (threadIdx.x & 63));
+  }
   march_rows<K, R, S>(kp, io, i0, jb, je, dt, dt_dx, dt_dy, r);
   if (io.epilogue) {
     const double m = wave_max(r.inv);
-    if ((threadIdx.x & 63) == 0) acc_max(io.acc, task, m);
+    if ((threadIdx.x & 63) == 0) acc_max(io.acc, slot, m);
   }
 }
-
 
 // How a stage of a single simulation gets its dt. The first stage of a step runs the loop control
 // itself: each of its waves takes the maximum over the slots of the previous state and forms the
@@ -187,16 +189,20 @@ __device__ inline bool march_begin(const MarchCtl &m, const KParams &kp, unsigne
 template <class K, typename R, typename S>
 __global__ void __launch_bounds__(64 * MARCH_WAVES) __attribute__((amdgpu_waves_per_eu(K::kWPE, K::kWPE)))
 march_kernel(const KParams kp, const StageIO<S> io, const MarchGeom g, const MarchCtl mc) {
-  // XCD x (blocks b with b % 8 == x) takes a contiguous run of blocks, so that neighbouring
-  // strips, which share halo columns, run on one L2
-  const int nb = gridDim.x, q = nb >> 3, rem = nb & 7;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // XCD x (blocks b with b % 8 == x) takes band x or, with one band, a contiguous run of blocks, so
+  // that neighbouring strips, which share halo columns, run on one L2
   const int x = blockIdx.x & 7, k = blockIdx.x >> 3;
-  const int blk = x * q + (x < rem ? x : rem) + k;
-  const int task = blk * MARCH_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (task >= g.ntasks) return;
+  const int q = gridDim.x >> 3, rem = gridDim.x & 7;
+  const int band = g.bands == 1 ? 0 : x;
+  const int t = (k + (g.bands == 1 ? x * q + (x < rem ? x : rem) : 0)) * MARCH_WAVES + w;
+  if (t >= g.per_band) return;
   double dt, dt_dx, dt_dy;
-  if (!march_begin(mc, kp, io.acc, task, dt, dt_dx, dt_dy)) return;  // the device loop has ended
-  march_task<K, R, S>(kp, io, g, task, dt, dt_dx, dt_dy);
+  // (the first band's first task records the step)
+  if (!march_begin(mc, kp, io.acc, band + t, dt, dt_dx, dt_dy)) return;  // the device loop has ended
+  int i0, jb, je;
+  march_task_rows(g, kp.Ny, band, t, i0, jb, je);
+  if (jb < je) march_task<K, R, S>(kp, io, i0, jb, je, t + 7 * band, dt, dt_dx, dt_dy);
 }
 
 // Batched stage: the waves of a persistent grid run the (job, task) pairs of one kernel class, each
@@ -231,8 +237,9 @@ batch_march_kernel(const BatchJob *__restrict__ jobs, const BatchItem *__restric
     StepCtl *ctl = J.ctl;
     if (task >= J.nblocks || !uni(ctl->active) || (!J.rk2 && stage == 2)) continue;
     const StageIO<S> io = batch_stage_io<S>(J, stage, uni(ctl->fresh), uni(ctl->nsteps));
-    const MarchGeom g = {J.nsx, J.nsy, J.seg, J.nblocks};
-    march_task<K, R, S>(J.kp, io, g, task, uni(ctl->dt), uni(ctl->dt_dx), uni(ctl->dt_dy));
+    const int sy = task / J.nsx, jb = sy * J.seg;  // uniform segments
+    march_task<K, R, S>(J.kp, io, (task - sy * J.nsx) * MARCH_OUT, jb, jb + J.seg < J.kp.Ny ? jb + J.seg : J.kp.Ny, task,
+                        uni(ctl->dt), uni(ctl->dt_dx), uni(ctl->dt_dy));
   }
 }
 
@@ -248,7 +255,7 @@ struct MarchLaunch {
   template <int RC, int RM, bool TC, bool VI, bool XG>
   hipError_t operator()() {
     typedef MarchStage<R, S, RC, RM, TC, VI, XG, DIVF> K;
-    hipLaunchKernelGGL((march_kernel<K, R, S>), dim3((g.ntasks + MARCH_WAVES - 1) / MARCH_WAVES),
+    hipLaunchKernelGGL((march_kernel<K, R, S>), dim3(g.bands * ((g.per_band + MARCH_WAVES - 1) / MARCH_WAVES)),
                        dim3(64 * MARCH_WAVES), 0, st, kp, io, g, mc);
     return hipGetLastError();
   }
@@ -295,6 +302,8 @@ hipError_t launch_march_fp64(const StageClass &c, const KParams &kp, const Stage
                              const MarchGeom &g, const MarchCtl &mc, hipStream_t st);
 hipError_t launch_march_fp64_exact(const StageClass &c, const KParams &kp, const StageIO<double> &io,
                              const MarchGeom &g, const MarchCtl &mc, hipStream_t st);
+hipError_t launch_march_fp32s64(const StageClass &c, const KParams &kp, const StageIO<double> &io,
+                                const MarchGeom &g, const MarchCtl &mc, hipStream_t st);
 hipError_t launch_march_fp32(const StageClass &c, const KParams &kp, const StageIO<float> &io,
                              const MarchGeom &g, const MarchCtl &mc, hipStream_t st);
 

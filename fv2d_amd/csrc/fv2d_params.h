@@ -152,10 +152,13 @@ inline int pick_seg_rows(const fv2d_params *p, int nw) {
 // every SIMD finishes together: at KH 2048^2 FP64 (S, us per step) 18: 235, 16 (9% into a second
 // round): 249. At most 40 rows, since the waves of one long round drift apart (KH 4096^2: one
 // round of 70 rows 930, two of 35 915).
+inline int march_slots(const fv2d_params *p) {  // resident waves per SIMD
+  const bool xg = p->gravity_mode || p->well_balanced_flux_at_y_bc || p->bctc_ymin || p->bctc_ymax;
+  return march_wpe(p->precision != FV2D_FP32, xg && (p->tc_active || p->visc_active));
+}
 inline int pick_march_rows(const fv2d_params *p) {
   const bool f64 = p->precision == FV2D_FP64;
-  const bool xg = p->gravity_mode || p->well_balanced_flux_at_y_bc || p->bctc_ymin || p->bctc_ymax;
-  const int simds = 1024, slots = march_wpe(f64, xg && (p->tc_active || p->visc_active));
+  const int simds = 1024, slots = march_slots(p);
   const double P = 0.95, L = f64 ? 2.3 : 1.1, I = f64 ? 1.5 : 0.55;
   const long long nsx = (p->Nx + MARCH_OUT - 1) / MARCH_OUT;
   int best = 40;
@@ -174,13 +177,34 @@ inline int pick_march_rows(const fv2d_params *p) {
   }
 }
 
+// Long-then-short split of the march kernel for grids with 8 or more rows per resident wave: every
+// wave of an XCD first gets `rounds` long segments (about 32 rows each) that leave 9% of a round's
+// rows over, which then run as short ones, so that a launch ends in a short segment's time however the
+// waves drift. Against uniform segments (us per step): KH 4096^2 FP64 888 -> 878, FP32 355 -> 340, KH
+// 2048^2 224 -> 217, 92 -> 87, Sedov 2048^2 FP64 224 -> 203, RT 1024x3072 151 -> 148. Fewer rows per
+// wave than that leave nothing to split (RT in segments of 16 and 8 rows at 13.5 a wave: 145, but
+// Sedov 2048^2 the same way 231).
+inline bool march_long_short(const fv2d_params *p, MarchGeom &g) {
+  const int waves = 128 * march_slots(p);  // per XCD
+  const int nsx = (p->Nx + MARCH_OUT - 1) / MARCH_OUT, rows = (p->Ny + 7) / 8;
+  const double per_wave = (double)nsx * rows / waves;
+  int rounds = (int)(per_wave / 32.0 + 0.5);
+  if (rounds < 1) rounds = 1;
+  const long long nl = (long long)rounds * waves / nsx;  // long segments per band
+  if (per_wave < 8.0 || nl < 1) return false;
+  const int seg = (int)((double)rows / nl * (1.0 - 0.09 / rounds));
+  if (seg < 8) return false;
+  const int sseg = seg / 5 > 4 ? seg / 5 : 4;
+  g = march_geom_banded(p->Nx, p->Ny, (int)nl, seg, sseg);
+  return true;
+}
+
 // Work split of the march kernel, the single-grid kernel unless chunk_rows asks for the strip
-// kernel (ntasks = 0). The FP32 form on an FP64 state also takes the strip kernel: it is held by
-// memory traffic, and the march, which reads U of a row again at its update, takes 680 us per step
-// at KH 4096^2 against 627.
+// kernel (ntasks = 0).
 inline MarchGeom sim_march_geom(const fv2d_params *p) {
-  MarchGeom g = {0, 0, 0, 0};
-  if (p->chunk_rows > 0 || p->precision == FV2D_FP32_STATE64) return g;
+  MarchGeom g = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (p->chunk_rows > 0) return g;
+  if (p->seg_rows <= 0 && march_long_short(p, g)) return g;
   return march_geom(p->Nx, p->Ny, p->seg_rows > 0 ? p->seg_rows : pick_march_rows(p));
 }
 

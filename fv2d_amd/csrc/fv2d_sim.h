@@ -143,7 +143,8 @@ inline hipError_t sim_launch_stage(SimDev &d, const void *src, int qsrc, const v
     io.qsrc = qsrc;
     io.epilogue = epilogue;
     if (sim_fp32s64(d))
-      e = launch_stage_fp32s64(d.kp, io, d.geom, recon, d.p.riemann_solver, tc, visc, d.stream);
+      e = d.march.ntasks ? launch_march_fp32s64(cls, d.kp, io, d.march, mc, d.stream)
+                         : launch_stage_fp32s64(d.kp, io, d.geom, recon, d.p.riemann_solver, tc, visc, d.stream);
     else
       e = d.march.ntasks ? launch_march_fp64(cls, d.kp, io, d.march, mc, d.stream)
                          : launch_stage_fp64(d.kp, io, d.geom, recon, d.p.riemann_solver, tc, visc, d.stream);

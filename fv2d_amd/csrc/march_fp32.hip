@@ -1,4 +1,5 @@
-// march_fp32.hip -- FP32-form instantiations of the register-march stage (U stored in FP32).
+// march_fp32.hip -- FP32-form instantiations of the register-march stage (U stored in FP32); those on
+// the FP64 state are in march_fp32s64.hip.
 #include "fv2d_march_device.h"
 
 namespace fv2d {

@@ -20,6 +20,7 @@ void march_run(Sim &s, const StageIO<S> &io) {
   typedef typename K::Lane Lane;
   std::vector<Lane> L(64);
   std::vector<R> low((size_t)K::NLOW * 64);
+  std::vector<S> ring((size_t)K::NRING * 64);
   double best = 0.0;
 #define EACH(stmt)                                                                                                     \
   for (int lane = 0; lane < 64; ++lane) {                                                                              \
@@ -32,11 +33,14 @@ void march_run(Sim &s, const StageIO<S> &io) {
 #define SHL(dst, src) EACH(r.dst = lane < 63 ? L[lane + 1].src : R(0))
   for (int task = 0; task < g.ntasks; ++task) {
     int i0, jb, je;
-    march_task_rows(g, kp.Ny, task, i0, jb, je);
+    march_task_rows(g, kp.Ny, task / g.per_band, task % g.per_band, i0, jb, je);
+    if (jb >= je) continue;
     for (auto &x : low) x = std::numeric_limits<R>::quiet_NaN();
+    for (auto &x : ring) x = std::numeric_limits<S>::quiet_NaN();
     for (int lane = 0; lane < 64; ++lane) {
       memset((void *)&L[lane], 0xff, sizeof(Lane));
       L[lane].low = low.data() + lane;
+      L[lane].ring = K::kRing ? ring.data() + lane : nullptr;
       K::set_column(lane, i0, kp, L[lane]);
     }
     for (int lane = 0; lane < 64; ++lane) {
@@ -134,3 +138,14 @@ void march_stage(Sim &s, const StageIO<S> &io) {
 
 #define stage_nw march_stage
 #include "tile_emu.cpp"
+
+// Tasks of the split the march kernel takes for these parameters: returns their number and fills (i0,
+// jb, je) of each into out (when not NULL); bands into *bands.
+extern "C" int emu_march_tasks(const fv2d_params *p, int *out, int *bands) {
+  const MarchGeom g = sim_march_geom(p);
+  *bands = g.bands;
+  if (out)
+    for (int t = 0; t < g.ntasks; ++t)
+      march_task_rows(g, p->Ny, t / g.per_band, t % g.per_band, out[3 * t], out[3 * t + 1], out[3 * t + 2]);
+  return g.ntasks;
+}

@@ -8,11 +8,12 @@ import os
 import subprocess
 import sys
 
+import numpy as np
 import pytest
 
 import emu as EMU
 import test_emulated_kernel as T
-from fv2d_amd.capi import PLM, Params
+from fv2d_amd.capi import FP32, FP32_STATE64, FP64, PLM, Params
 
 HERE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "emu")
 FLAGS = ["-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", "-fno-fast-math", "-Wno-unknown-pragmas"]
@@ -65,6 +66,29 @@ def test_grid_shapes_bitwise(Nx, Ny, seg, march_lib, oracle_lib):
     for n, c in enumerate(CLASSES):
         p, q0 = T.make(n, *c, Nx=Nx, Ny=Ny)
         T.compare(p.copy(seg_rows=seg), q0, march_lib, oracle_lib, steps=2)
+
+
+@pytest.mark.parametrize("precision", [FP64, FP32, FP32_STATE64])
+@pytest.mark.parametrize("Nx,Ny,seg,banded", [
+    (2, 2, 0, False), (512, 8, 0, False), (1024, 1024, 0, False), (60, 70, 4, False), (4096, 4096, 0, True),
+    (2048, 2048, 0, True), (4097, 4099, 0, True), (60, 40001, 0, None), (70000, 301, 0, True), (2048, 2048, 64, False)])
+def test_tasks_cover_the_grid_once(Nx, Ny, seg, banded, precision, march_lib):
+    """Every (strip, row) belongs to one task, in the uniform and in the banded long-then-short split."""
+    p = Params.defaults(Nx=Nx, Ny=Ny, seg_rows=seg, precision=precision)
+    march_lib.emu_march_tasks.argtypes = [C.POINTER(Params), C.POINTER(C.c_int), C.POINTER(C.c_int)]
+    bands = C.c_int()
+    n = march_lib.emu_march_tasks(C.byref(p), None, C.byref(bands))
+    out = np.zeros((n, 3), dtype=np.int32)
+    march_lib.emu_march_tasks(C.byref(p), out.ctypes.data_as(C.POINTER(C.c_int)), C.byref(bands))
+    if banded is not None:  # (60 x 40001: 10 rows per wave of an FP64 grid, 6.5 of an FP32 one)
+        assert bands.value == (8 if banded else 1)
+    live = out[out[:, 2] > out[:, 1]]
+    assert (live[:, 0] % 60 == 0).all() and live[:, 0].max() < Nx and live[:, 1].min() == 0 and live[:, 2].max() == Ny
+    nsx = -(-Nx // 60)
+    edge = np.zeros((nsx, Ny + 1), dtype=np.int64)
+    np.add.at(edge, (live[:, 0] // 60, live[:, 1]), 1)
+    np.add.at(edge, (live[:, 0] // 60, live[:, 2]), -1)
+    assert (np.cumsum(edge, axis=1)[:, :Ny] == 1).all()
 
 
 def test_resets_nan_and_fp32(march_lib, oracle_lib):
