@@ -4,13 +4,14 @@
 //  - device memory: one arena allocated at creation; a job takes one contiguous range of it
 //    (U, Us, Q0 planes with the single-simulation layout, its dt partials, its gravity row)
 //    and gets it back when collected. Admission = a free slot + a free range (first fit).
-//  - control: one StepCtl per slot on the device. Each step, batch_reduce_kernel reduces
-//    every running job's dt partials and runs its loop control (the same advance_control as
-//    the single-simulation path), so jobs at different steps, with different dt, advance in
+//  - control: one StepCtl per slot on the device. Each step, batch_control_kernel (march classes;
+//    batch_reduce_kernel for strip classes) takes every running job's dt maximum and runs its loop
+//    control (the same advance_control as the single-simulation path), so jobs at different steps, with different dt, advance in
 //    the same launches and stop on the device at their own end.
-//  - work list: pack_items_kernel lists (slot, strip segment) items per kernel class
-//    (reconstruction, Riemann solver, conduction, viscosity, wall/gravity variant); the
-//    persistent batch_stage_kernel of each class pulls items from its run of the list.
+//  - work list: pack_items_kernel lists (slot, strip segment) or (slot, group of march tasks) items
+//    per kernel class (reconstruction, Riemann solver, conduction, viscosity, wall/gravity variant,
+//    strip or march kernel); the persistent kernel of each class pulls its work from its run of the
+//    list (batch_march_kernel: wave by wave).
 //  - launches: each kernel class runs its own chain of steps_per_launch steps (reduce, stage
 //    1, stage 2) on a stream of its own, forked from and joined back into the batch stream,
 //    so that the drain of one class's persistent kernel overlaps the others' work. The

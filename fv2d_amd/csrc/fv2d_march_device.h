@@ -18,7 +18,7 @@ __device__ inline float shr1(float x) { return __int_as_float(dpp_shr(__float_as
 __device__ inline float shl1(float x) { return __int_as_float(dpp_shl(__float_as_int(x))); }
 // shl1 that leaves lane 63 its own value (in place when x dies here): a face state between real
 // states keeps that lane off the division and square-root fallbacks, which the whole wave would
-// run with it.
+// run with it (Sedov 2048^2 FP64: 245 us per step with a zero state there, 230 without).
 __device__ inline double shl1_keep(double x) {
   const int lo = __double2loint(x), hi = __double2hiint(x);
   return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, 0x130, 0xf, 0xf, false),
@@ -30,7 +30,8 @@ __device__ inline float shl1_keep(float x) {
 }
 
 // Slots parked in LDS must stay there: without this the compiler forwards every stored value to
-// its read of the next row in registers, which it then spills to scratch.
+// its read of the next row in registers, which it then spills to scratch (KH FP64: 20 registers
+// spilled, 1019 us per step at 4096^2; none, 927).
 template <typename R>
 __device__ inline LanePtr<R> opaque(LanePtr<R> p) {
 #if defined(__HIP_DEVICE_COMPILE__)

@@ -139,8 +139,8 @@ struct Ops<float> {
 // equal, so every quotient has the bits of a / b (and is a / b when they differ).
 // v_div_scale gives NaN for a zero or NaN operand, and v_div_fixup then sets the quotient from a
 // and b alone (signed zeros, infinities, NaNs): such a numerator also takes the short way. That
-// matters wherever a velocity is exactly zero (gas at rest, flow along one axis): sent to a / b
-// there, the quotients made the point blast's FP64 stage 14% slower.
+// matters wherever a velocity is exactly zero (gas at rest, flow along one axis): Sedov 2048^2 FP64
+// 256 us per step with such numerators sent to a / b, 245 this way.
 // On the host and in the FP32 form (where division is a * rcp(b), the reciprocal shared by the
 // compiler) it is plain division.
 template <typename R>

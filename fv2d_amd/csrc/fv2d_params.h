@@ -208,7 +208,7 @@ inline MarchGeom sim_march_geom(const fv2d_params *p) {
   return march_geom(p->Nx, p->Ny, p->seg_rows > 0 ? p->seg_rows : pick_march_rows(p));
 }
 
-// Strip geometry of the single-grid kernel: the banded long-then-short schedule when the
+// Strip geometry of the strip kernel on a single grid: the banded long-then-short schedule when the
 // uniform segments make at least 2048 workgroups (two rounds of 4 per CU on 256 CUs), else
 // the uniform one.
 inline StripGeom sim_geom(const fv2d_params *p) {

@@ -1,5 +1,6 @@
-// fv2d_stage.h -- the fused stage of the hydro step: column-strip marching, one wave per
-// row, one lane per column.
+// fv2d_stage.h -- what the two kernels of the fused hydro stage share (StageOps), and the strip
+// kernel: column-strip marching, one wave per row, one lane per column. The strip kernel runs where
+// chunk_rows asks for it; the march kernel (fv2d_march.h) is the default and the faster one.
 //
 // A workgroup of 4 wave64s owns a strip of 62 domain columns and a segment of rows, and
 // marches up the segment 4 rows (one "chunk") at a time. Lane l of every wave stands for
