@@ -87,9 +87,10 @@ __global__ void __launch_bounds__(256) batch_reduce_kernel(const BatchJob *jobs,
 }
 
 // Work list: for each class c, the items (slot, segment; march classes: slot, group of tasks) of
-// every used, running job of class c, in slot order, at items[ranges[2c] .. ranges[2c] + ranges[2c+1]).
+// every used, running job of class c, in slot order, at items[ranges[3c] .. ranges[3c] + ranges[3c+1]).
+// ranges[3c+2] = rows: the task height of the march jobs without a seg_rows of their own.
 __global__ void __launch_bounds__(1024) pack_items_kernel(const BatchJob *jobs, int nslots, int nclasses,
-                                                          BatchItem *items, int *ranges) {
+                                                          BatchItem *items, int *ranges, int rows) {
   __shared__ int cnt[MAX_SLOTS];
   const int s = threadIdx.x;
   int base = 0;
@@ -98,7 +99,7 @@ __global__ void __launch_bounds__(1024) pack_items_kernel(const BatchJob *jobs, 
     if (c < nclasses && s < nslots) {
       const BatchJob &J = jobs[s];
       if (J.used && J.cls == c && J.ctl->active)
-        n = J.march ? (J.nblocks + MARCH_GROUP - 1) / MARCH_GROUP : J.nblocks;
+        n = J.march ? (march_tasks(J, rows) + MARCH_GROUP - 1) / MARCH_GROUP : J.nblocks;
     }
     cnt[s] = n;
     __syncthreads();
@@ -117,8 +118,9 @@ __global__ void __launch_bounds__(1024) pack_items_kernel(const BatchJob *jobs, 
       items[start + b] = it;
     }
     if (s == 0) {
-      ranges[2 * c] = base;
-      ranges[2 * c + 1] = total;
+      ranges[3 * c] = base;
+      ranges[3 * c + 1] = total;
+      ranges[3 * c + 2] = rows;
     }
     base += total;
     __syncthreads();
@@ -187,13 +189,19 @@ StripGeom batch_geom(const fv2d_params *p) {
   return strip_geom(p->Nx, p->Ny, batch_seg_rows(p), batch_chunk_rows(p));
 }
 
-// The march kernel's split (jobs without chunk_rows): tasks of 16 rows by default. Its items of
-// MARCH_GROUP tasks are then never more than the strip split's (at most twice the strips, four
-// times the segments).
+// The march kernel's split (jobs without chunk_rows): tasks of seg_rows rows, or of the work list's
+// height (batch_rows), at most 16. Its items of MARCH_GROUP tasks are at 16 rows never more than the
+// strip split's (at most twice the strips, four times the segments).
 bool batch_march(const fv2d_params *p) { return p->chunk_rows <= 0; }
-MarchGeom batch_march_geom(const fv2d_params *p) {
-  return march_geom(p->Nx, p->Ny, p->seg_rows > 0 ? p->seg_rows : 16);
+// A segment taller than the grid counts as one of its height (task numbers times heights fit an int).
+int march_seg(const fv2d_params *p, int rows) {
+  return p->seg_rows <= 0 ? rows : p->seg_rows < p->Ny ? p->seg_rows : p->Ny;
 }
+
+// Items that the work list may hold beyond max_items: lists of less than 16 rows per task, which
+// batch_rows allows up to one task per resident wave, and a part-filled group per job.
+constexpr int BATCH_ROWS_TASKS = 6 * 1024;  // resident waves, at most 6 per SIMD
+constexpr int EXTRA_ITEMS = BATCH_ROWS_TASKS / MARCH_GROUP + MAX_SLOTS;
 
 JobLayout job_layout(const fv2d_params *p) {
   const size_t esize = (p->precision == FV2D_FP32) ? 4 : 8;
@@ -342,7 +350,7 @@ static hipError_t enqueue_class_step(fv2d_batch *b, int c, hipStream_t st) {
   const bool f32 = b->cfg.precision == FV2D_FP32;
   for (int stage = 1; stage <= 2; ++stage) {
     int *counter = b->d_counters + (2 * c + (stage - 1)) * COUNTER_WORDS;
-    const int *range = b->d_ranges + 2 * c;
+    const int *range = b->d_ranges + 3 * c;
     e = f32 ? launch_batch_fp32(b->classes[c], b->d_jobs, b->d_items, range, counter, stage, b->grid[c], st)
             : launch_batch_fp64(b->classes[c], b->d_jobs, b->d_items, range, counter, stage, b->grid[c], st);
     if (e != hipSuccess) return e;
@@ -498,9 +506,9 @@ int fv2d_batch_create(const fv2d_batch_config *c, fv2d_batch **out) {
   if ((e = hipMalloc((void **)&b->d_ctl, sizeof(StepCtl) * c->max_jobs)) != hipSuccess) return fail("ctl", e);
   if ((e = hipMalloc((void **)&b->d_acc, sizeof(unsigned long long) * ACC_WORDS * c->max_jobs)) != hipSuccess)
     return fail("dt slots", e);
-  if ((e = hipMalloc((void **)&b->d_items, sizeof(BatchItem) * (size_t)c->max_items)) != hipSuccess)
+  if ((e = hipMalloc((void **)&b->d_items, sizeof(BatchItem) * ((size_t)c->max_items + EXTRA_ITEMS))) != hipSuccess)
     return fail("work list", e);
-  if ((e = hipMalloc((void **)&b->d_ranges, sizeof(int) * 2 * MAX_CLASSES)) != hipSuccess) return fail("ranges", e);
+  if ((e = hipMalloc((void **)&b->d_ranges, sizeof(int) * 3 * MAX_CLASSES)) != hipSuccess) return fail("ranges", e);
   if ((e = hipMalloc((void **)&b->d_counters, sizeof(int) * 2 * MAX_CLASSES * COUNTER_WORDS)) != hipSuccess)
     return fail("counters", e);
   if ((e = hipMalloc((void **)&b->d_sums, sizeof(double) * 4)) != hipSuccess) return fail("sums", e);
@@ -512,7 +520,7 @@ int fv2d_batch_create(const fv2d_batch_config *c, fv2d_batch **out) {
     return fail("clear jobs", e);
   if ((e = hipMemsetAsync(b->d_ctl, 0, sizeof(StepCtl) * c->max_jobs, b->stream)) != hipSuccess)
     return fail("clear ctl", e);
-  if ((e = hipMemsetAsync(b->d_ranges, 0, sizeof(int) * 2 * MAX_CLASSES, b->stream)) != hipSuccess)
+  if ((e = hipMemsetAsync(b->d_ranges, 0, sizeof(int) * 3 * MAX_CLASSES, b->stream)) != hipSuccess)
     return fail("clear ranges", e);
   if ((e = hipMemsetAsync(b->d_counters, 0, sizeof(int) * 2 * MAX_CLASSES * COUNTER_WORDS, b->stream)) != hipSuccess)
     return fail("clear counters", e);
@@ -638,11 +646,8 @@ int fv2d_batch_submit(fv2d_batch *b, const fv2d_params *p, const fv2d_problem *p
   dj.nsx = J.g.nsx;
   dj.nsy = J.g.nsy;
   if (batch_march(p)) {
-    const MarchGeom mg = batch_march_geom(p);
-    dj.nblocks = mg.ntasks;
-    dj.seg = mg.seg;
-    dj.nsx = mg.nsx;
-    dj.nsy = mg.ntasks / mg.nsx;
+    dj.seg = march_seg(p, 0);
+    dj.nsx = march_strips(p->Nx);
     dj.march = 1;
   }
   dj.U = J.U;
@@ -672,13 +677,47 @@ int fv2d_batch_submit(fv2d_batch *b, const fv2d_params *p, const fv2d_problem *p
   return FV2D_OK;
 }
 
+// Task height of the march jobs without seg_rows: 16, or less while the jobs in the batch would leave
+// SIMDs idle or short of waves. Estimate and constants of pick_march_rows with the tasks of all jobs
+// together; below 16 rows only up to one task per resident wave, where each row of a task costs time
+// but an empty SIMD costs nothing. KH 128^2, us per step at 16 rows and by this rule: 64 jobs FP32 71 ->
+// 51, FP64 149 -> 117; 4 jobs 55 -> 23, 105 -> 39. Lists of more tasks than waves keep 16 rows (96 jobs of
+// 128^2 to 1M cells, FP32: 16 rows 690, 8 rows 730).
+static int batch_rows(const fv2d_batch *b) {
+  const bool f64 = b->cfg.precision == FV2D_FP64;
+  const int slots = march_wpe(f64, false);
+  int best = 16;
+  double best_t = 1e300;
+  for (int rows = 16; rows >= 4; rows /= 2) {
+    long long tasks = 0;
+    for (const JobHost &J : b->slots) {
+      if (J.status != FV2D_JOB_RUNNING) continue;
+      if (!batch_march(&J.p))
+        tasks += (long long)J.g.nblocks * batch_chunk_rows(&J.p);  // waves
+      else {
+        const int seg = march_seg(&J.p, rows);
+        tasks += (long long)march_strips(J.p.Nx) * ((J.p.Ny + seg - 1) / seg);
+      }
+    }
+    if (rows < 16 && tasks > 1024 * slots) break;
+    const double w = tasks > 1024 * slots ? slots : (double)((tasks + 1023) / 1024);
+    const double rounds = tasks > 1024 * slots ? (double)tasks / (1024 * slots) : 1.0;
+    const double t = march_time(f64, rows, w) * rounds;
+    if (t < best_t) {
+      best = rows;
+      best_t = t;
+    }
+  }
+  return best;
+}
+
 int fv2d_batch_launch(fv2d_batch *b, int32_t launches) {
   if (!b) return FV2D_E_INVALID;
   if (launches < 1) BFAIL(b, FV2D_E_INVALID, "fv2d_batch_launch: launches must be >= 1");
   BHIP(b, hipSetDevice(b->device));
   if (b->dirty) {
     hipLaunchKernelGGL(pack_items_kernel, dim3(1), dim3(MAX_SLOTS), 0, b->stream, b->d_jobs, b->cfg.max_jobs,
-                       (int)b->classes.size(), b->d_items, b->d_ranges);
+                       (int)b->classes.size(), b->d_items, b->d_ranges, batch_rows(b));
     BHIP(b, hipGetLastError());
     b->dirty = false;
   }

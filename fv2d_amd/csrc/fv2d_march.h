@@ -46,9 +46,11 @@ struct MarchGeom {
   int ntasks;    // bands * per_band
 };
 
+FV2D_HD constexpr int march_strips(int Nx) { return (Nx + MARCH_OUT - 1) / MARCH_OUT; }
+
 FV2D_HD MarchGeom march_geom(int Nx, int Ny, int seg) {
   MarchGeom g;
-  g.nsx = (Nx + MARCH_OUT - 1) / MARCH_OUT;
+  g.nsx = march_strips(Nx);
   g.bands = 1;
   g.height = Ny;
   g.nlong = (Ny + seg - 1) / seg;

@@ -215,11 +215,17 @@ march_kernel(const KParams kp, const StageIO<S> io, const MarchGeom g, const Mar
 // learn that nothing is left. Waves do not wait for each other. stage as in batch_stage_kernel.
 constexpr int MARCH_GROUP = 8;
 
+// Tasks of a march job; rows: the work list's height.
+__device__ inline int march_tasks(const BatchJob &J, int rows) {
+  const int seg = J.seg > 0 ? J.seg : rows;
+  return J.nsx * ((J.kp.Ny + seg - 1) / seg);
+}
+
 template <class K, typename R, typename S>
 __global__ void __launch_bounds__(64 * MARCH_WAVES) __attribute__((amdgpu_waves_per_eu(K::kWPE, K::kWPE)))
 batch_march_kernel(const BatchJob *__restrict__ jobs, const BatchItem *__restrict__ items, const int *range,
                    int *counter, int stage) {
-  const int base = range[0], n = range[1] * MARCH_GROUP;
+  const int base = range[0], n = range[1] * MARCH_GROUP, rows = range[2];
   const int x = blockIdx.x & 7;
   const int lo = (int)((long long)n * x >> 3), hi = (int)((long long)n * (x + 1) >> 3);
   const int waves = ((int)(gridDim.x + 7 - x) >> 3) * MARCH_WAVES;  // of this XCD
@@ -236,10 +242,11 @@ batch_march_kernel(const BatchJob *__restrict__ jobs, const BatchItem *__restric
     const BatchJob &J = jobs[uni(wi.job)];
     const int task = uni(wi.blk) * MARCH_GROUP + it % MARCH_GROUP;
     StepCtl *ctl = J.ctl;
-    if (task >= J.nblocks || !uni(ctl->active) || (!J.rk2 && stage == 2)) continue;
+    const int seg = J.seg > 0 ? J.seg : rows;
+    const int sy = task / J.nsx, jb = sy * seg;  // uniform segments
+    if (jb >= J.kp.Ny || !uni(ctl->active) || (!J.rk2 && stage == 2)) continue;
     const StageIO<S> io = batch_stage_io<S>(J, stage, uni(ctl->fresh), uni(ctl->nsteps));
-    const int sy = task / J.nsx, jb = sy * J.seg;  // uniform segments
-    march_task<K, R, S>(J.kp, io, (task - sy * J.nsx) * MARCH_OUT, jb, jb + J.seg < J.kp.Ny ? jb + J.seg : J.kp.Ny, task,
+    march_task<K, R, S>(J.kp, io, (task - sy * J.nsx) * MARCH_OUT, jb, jb + seg < J.kp.Ny ? jb + seg : J.kp.Ny, task,
                         uni(ctl->dt), uni(ctl->dt_dx), uni(ctl->dt_dy));
   }
 }

@@ -156,11 +156,14 @@ inline int march_slots(const fv2d_params *p) {  // resident waves per SIMD
   const bool xg = p->gravity_mode || p->well_balanced_flux_at_y_bc || p->bctc_ymin || p->bctc_ymax;
   return march_wpe(p->precision != FV2D_FP32, xg && (p->tc_active || p->visc_active));
 }
+inline double march_time(bool f64, int S, double w) {
+  const double P = 0.95, L = f64 ? 2.3 : 1.1, I = f64 ? 1.5 : 0.55;
+  return (S + P) * sqrt(L * L + w * w * I * I);
+}
 inline int pick_march_rows(const fv2d_params *p) {
   const bool f64 = p->precision == FV2D_FP64;
   const int simds = 1024, slots = march_slots(p);
-  const double P = 0.95, L = f64 ? 2.3 : 1.1, I = f64 ? 1.5 : 0.55;
-  const long long nsx = (p->Nx + MARCH_OUT - 1) / MARCH_OUT;
+  const long long nsx = march_strips(p->Nx);
   int best = 40;
   double best_t = 1e300;
   for (int k = 1;; ++k) {
@@ -168,7 +171,7 @@ inline int pick_march_rows(const fv2d_params *p) {
     const long long nsy = (long long)simds * w * rounds / nsx;
     if (nsy < 1) continue;
     const int S = (int)((p->Ny + nsy - 1) / nsy);
-    const double t = (S + P) * rounds * sqrt(L * L + w * w * I * I);
+    const double t = march_time(f64, S, w) * rounds;
     if (S <= 40 && t < best_t) {
       best = S;
       best_t = t;

@@ -74,8 +74,8 @@ struct StageIO {
 // precision; buffers are typed by it.
 struct BatchJob {
   KParams kp;
-  int nblocks;   // workgroup items of this job (strip geometry), or wave tasks (march)
-  int seg;       // rows per segment
+  int nblocks;   // workgroup items of this job (strip geometry)
+  int seg;       // rows per segment; march: of a task, 0 = the work list's height
   int nsx, nsy;
   int march;     // the class runs the march kernel
   void *U, *Us, *Q0;

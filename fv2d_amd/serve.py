@@ -270,7 +270,7 @@ def fifo_latencies(specs: list[JobSpec], service: dict) -> np.ndarray:
 
 # Tile candidates of the batched stage kernels: (segment height = rows per work item, chunk rows:
 # 0 the march kernel, 4 or 8 the strip kernel with that many waves per workgroup).
-TILE_CANDIDATES = ((16, 0), (8, 0), (24, 0), (32, 0), (64, 4))
+TILE_CANDIDATES = ((0, 0), (8, 0), (24, 0), (32, 0), (64, 4))
 
 
 def _time_batch(specs_params, config: BatchConfig, launches: int = 3, warm: int = 1, lib=None) -> float:
@@ -290,7 +290,7 @@ def _time_batch(specs_params, config: BatchConfig, launches: int = 3, warm: int 
 
 
 def autotune(precision: int = FP32, sizes=SERVE_SIZES, kinds=KINDS, target_cells: int = 12 << 20,
-             tiles=TILE_CANDIDATES, blocks_per_cu=(0, 3, 2), mix_tiles=((16, 0), (24, 0), (64, 4)), cache: str | None = None,
+             tiles=TILE_CANDIDATES, blocks_per_cu=(0, 3, 2), mix_tiles=((0, 0), (24, 0), (64, 4)), cache: str | None = None,
              lib=None, log=None, use_graph: int = 1) -> dict:
     """Choose the tile of the batched stage kernel per kernel class (setup) and grid: the
     segment height (rows per work item) and the chunk height (rows per chunk = waves per
