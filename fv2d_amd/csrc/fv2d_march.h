@@ -8,9 +8,9 @@
 // is no LDS and no barrier: waves never wait for each other, so a SIMD always has other waves
 // to issue from, and every interface is solved once. What a row needs late (the lower face's terms,
 // the next row's left states, FP64: row j+2) waits in slots of LDS that only the lane itself uses.
-// Bound by VALU issue: KH 4096^2 (PLM, HLLC, conduction, viscosity) FP64 690 VALU instructions per
-// cell and stage, 85% busy over the launch, 878 us per step (strip kernel: 742, 75%, 1020); FP32 366,
-// 98%, 342 us (389, 96%, 405). Per row j:
+// Bound by VALU issue: KH 4096^2 (PLM, HLLC, conduction, viscosity) FP64 697 VALU instructions per
+// cell and stage, 88% busy over the launch, 890 us per step (strip kernel: 742, 75%, 1020); FP32 365,
+// always busy, 345 us (389, 96%, 405). Per row j:
 //   begin   row j+2 from storage values (loaded one row ahead) to primitives
 //   diffs   differences along x, from column l+1            (shift: primitives of row j)
 //   slopes  minmod slopes and face states of x (row j) and y (row j+1)   (shift: differences)
